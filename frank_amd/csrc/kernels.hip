@@ -6,10 +6,9 @@
 //    lane l holds rows l + 64*t.  Column reductions are DPP / swizzle /
 //    permlane butterflies (bitwise identical in every lane); the only workgroup
 //    barrier per Householder step publishes the reflector through LDS.
-//  * Jacobi SVD of the K x K core: for K <= 16 one wave keeps the core in
-//    VGPRs (a lane group per column pair, columns moved between pairs by DPP
-//    wave shifts); larger cores run in LDS, QR-preconditioned, with a
-//    round-robin pairing so K/2 rotations proceed in parallel.
+//  * Jacobi SVD of the K x K core in LDS, a lane group per column pair,
+//    preconditioned by a pivoted QR held in VGPRs, with a round-robin pairing
+//    so K/2 rotations proceed in parallel.
 //  * Column-pivoted QR streams the tile through L2 with one thread per column
 //    (row-major tiles => every row sweep is coalesced).
 #include <hip/hip_runtime.h>
@@ -1745,516 +1744,6 @@ void launch_tri_extract(const T* src, int64_t rs, int64_t cs, T* dst, int64_t ld
 // ===========================================================================
 // One-sided (Hestenes) Jacobi SVD of the K x K core with truncation.
 // ===========================================================================
-// Rotation (c, s) that zeroes the off-diagonal of [[al, ga], [ga, be]]
-// (Rutishauser's formulas: t = sign(zeta) / (|zeta| + sqrt(1 + zeta^2)),
-// zeta = (be - al) / (2 ga), c = 1 / sqrt(1 + t^2), s = c t).  FP32 uses the
-// hardware reciprocal, square root and reciprocal square root (about 1 ulp: the rotation
-// stays orthogonal to rounding level, only its angle moves by an ulp); FP64
-// keeps the correctly rounded operations.
-__device__ __forceinline__ void jacobi_rotation(float al, float be, float ga, float& c, float& s) {
-  const float zeta = (be - al) * __builtin_amdgcn_rcpf(2.0f * ga);
-  const float t = copysignf(1.0f, zeta) * __builtin_amdgcn_rcpf(fabsf(zeta) + __builtin_amdgcn_sqrtf(1.0f + zeta * zeta));
-  c = __builtin_amdgcn_rsqf(1.0f + t * t);
-  s = c * t;
-}
-__device__ __forceinline__ void jacobi_rotation(double al, double be, double ga, double& c, double& s) {
-  const double zeta = (be - al) / (2.0 * ga);
-  const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-  c = 1.0 / sqrt(1.0 + t * t);
-  s = c * t;
-}
-
-__device__ __forceinline__ int rr_pos(int pos, int r, int k2) {
-  return pos == 0 ? 0 : ((pos - 1 + r) % (k2 - 1)) + 1;
-}
-
-template <typename T, int KMAX, int NT, bool VG, class Src>
-__global__ __launch_bounds__(NT) void svd_kernel(Src items) {
-  const SvdItem it = items.get(blockIdx.x);
-  const int K = it.K;
-  __shared__ T G[KMAX][KMAX + 1];
-  // right vectors: LDS, or a K x K global scratch (column j at vg + j * K) when they do not fit
-  __shared__ T Vs[VG ? 1 : KMAX][KMAX + 1];
-  __shared__ T coef[KMAX];
-  __shared__ int accept_sh;
-  T* vg = static_cast<T*>(it.vwork);
-  auto VA = [&](int j, int row) -> T& {
-    if constexpr (VG)
-      return vg[(int64_t)j * K + row];
-    else
-      return Vs[j][row];
-  };
-  __shared__ T sig[KMAX];
-  __shared__ int order[KMAX];
-  __shared__ int rank_sh;
-  // QR preconditioning (Drmac-Veselic): M P = Q R by column-pivoted Householder,
-  // then one-sided Jacobi on R^T, whose graded rows converge in few sweeps.  Q is
-  // formed in the right-vector array before the rotations, which then turn it
-  // into the left vectors, unless the right vectors live in global memory (VG:
-  // the left vectors are then formed as M v / sigma).  Every variant
-  // preconditions (the flag marks the preconditioning code).
-  constexpr bool PRE = true;
-  __shared__ int perm[KMAX];
-  __shared__ T tauq[KMAX];
-  __shared__ T cnorm[KMAX];
-  __shared__ int piv_sh;
-  const int tid = threadIdx.x;
-  if (K <= 0) {
-    if (tid == 0 && it.rank_out) *it.rank_out = 0;
-    return;
-  }
-  if constexpr (VG) {
-    if (vg == nullptr) {  // missing scratch: report an impossible rank instead of touching memory
-      if (tid == 0 && it.rank_out) *it.rank_out = -(1 << 20);
-      return;
-    }
-  }
-  if (it.mode == 0) {
-    for (int e = tid; e < K * K; e += NT) {
-      const int i = e / K, j = e % K;
-      G[j][i] = static_cast<const T*>(it.M)[i * it.m_rs + j * it.m_cs];
-      VA(j, i) = (i == j) ? T(1) : T(0);
-    }
-  } else {
-    // stage Ru (K x J) into G and Rv (K x J) into Vs with independent loads
-    const int J = it.kx;
-    const T* Ru = static_cast<const T*>(it.Ru);
-    const T* Rv = static_cast<const T*>(it.Rv);
-    for (int e = tid; e < K * J; e += NT) {
-      const int i = e / J, t = e % J;
-      G[t][i] = Ru[i * it.ldr + t];
-      VA(t, i) = Rv[i * it.ldr + t];
-    }
-    __syncthreads();
-    constexpr int PER = (KMAX * KMAX + NT - 1) / NT;
-    T mv[PER];
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int e = tid + u * NT;
-      T sacc = T(0);
-      if (e < K * K) {
-        const int i = e / K, j = e % K;
-        for (int t = 0; t < J; ++t) sacc += G[t][i] * VA(t, j);
-        if (i < it.ka && j < it.ka) sacc += static_cast<const T*>(it.Sa)[i * it.lds_in + j];
-      }
-      mv[u] = sacc;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int e = tid + u * NT;
-      if (e < K * K) {
-        const int i = e / K, j = e % K;
-        G[j][i] = mv[u];
-        VA(j, i) = (i == j) ? T(1) : T(0);
-      }
-    }
-  }
-  __syncthreads();
-  // Scale by a power of two so that max |M_ij| lies in [1, 2): exact, and it
-  // keeps squared column norms clear of underflow in the rotation tests.
-  using UB = typename std::conditional<sizeof(T) == 8, unsigned long long, unsigned int>::type;
-  __shared__ UB amax_bits;
-  __shared__ T tiny_sh;
-  if (tid == 0) amax_bits = 0;
-  __syncthreads();
-  {
-    T mx = T(0);
-    for (int e = tid; e < K * K; e += NT) mx = fmax(mx, fabs(G[e / K][e % K]));
-    UB bits;
-    memcpy(&bits, &mx, sizeof(T));
-    atomicMax(&amax_bits, bits);
-  }
-  __syncthreads();
-  T amax;
-  {
-    const UB bits = amax_bits;
-    memcpy(&amax, &bits, sizeof(T));
-  }
-  int sexp = 0;
-  if (amax > T(0) && isfinite(amax)) sexp = ilogb(amax);
-  const T scale = ldexp(T(1), -sexp), unscale = ldexp(T(1), sexp);
-  for (int e = tid; e < K * K; e += NT) G[e / K][e % K] *= scale;
-  __syncthreads();
-  if constexpr (VG) {
-    // the rotations' vectors do not fit in LDS: the sweeps rotate only G, and
-    // the kept left vectors are formed afterwards as M P g_c / sigma_c from this
-    // copy of the (scaled) matrix, column j at vg + j K
-    for (int e = tid; e < K * K; e += NT) vg[(int64_t)(e / K) * K + e % K] = G[e / K][e % K];
-    __syncthreads();
-  }
-  if constexpr (PRE) {
-    for (int c = tid; c < K; c += NT) perm[c] = c;
-    __syncthreads();
-    // gq lanes of one wave per column (rows split between them)
-    int gq = 64;
-    while (gq > 1 && K * gq > NT) gq >>= 1;
-    const int qc = tid / gq, qg = tid % gq;
-    for (int j = 0; j < K; ++j) {
-      // pivot: the column of largest norm over rows j..K-1
-      for (int c0 = j; c0 < K; c0 += NT / gq) {
-        const int c = c0 + qc;
-        T q = T(0);
-        if (c < K)
-          for (int row = j + qg; row < K; row += gq) q += G[c][row] * G[c][row];
-        q = group_sum(q, gq);
-        if (c < K && qg == 0) cnorm[c] = q;
-      }
-      __syncthreads();
-      if (tid == 0) {
-        int pv = j;
-        for (int c = j + 1; c < K; ++c)
-          if (cnorm[c] > cnorm[pv]) pv = c;
-        piv_sh = pv;
-        if (pv != j) {
-          const int t0 = perm[j];
-          perm[j] = perm[pv];
-          perm[pv] = t0;
-        }
-      }
-      __syncthreads();
-      const int pv = piv_sh;
-      if (pv != j)
-        for (int row = tid; row < K; row += NT) {
-          const T a = G[j][row];
-          G[j][row] = G[pv][row];
-          G[pv][row] = a;
-        }
-      __syncthreads();
-      // Householder reflector of column j below its diagonal (LAPACK dlarfg)
-      if (tid < 64) {
-        T q = T(0);
-        for (int row = j + 1 + tid; row < K; row += 64) q += G[j][row] * G[j][row];
-        q = wave_sum(q);
-        if (tid == 0) {
-          const T alpha = G[j][j];
-          T tau = T(0), beta = alpha, inv = T(0);
-          if (q > T(0)) {
-            beta = (alpha >= T(0) ? T(-1) : T(1)) * sqrt(alpha * alpha + q);
-            tau = (beta - alpha) / beta;
-            inv = T(1) / (alpha - beta);
-          }
-          tauq[j] = tau;
-          cnorm[j] = inv;  // the scaling of v below the diagonal
-          G[j][j] = beta;
-        }
-      }
-      __syncthreads();
-      const T inv = cnorm[j], tau = tauq[j];
-      for (int row = j + 1 + tid; row < K; row += NT) G[j][row] *= inv;
-      __syncthreads();
-      // apply H_j to the trailing columns: x -= tau v (v^T x), v = [1; G[j][j+1..]]
-      if (tau != T(0))
-        for (int c0 = j + 1; c0 < K; c0 += NT / gq) {
-          const int c = c0 + qc;
-          T w = T(0);
-          if (c < K) {
-            if (qg == 0) w = G[c][j];
-            for (int row = j + 1 + qg; row < K; row += gq) w += G[j][row] * G[c][row];
-          }
-          w = group_sum(w, gq) * tau;
-          if (c < K) {
-            if (qg == 0) G[c][j] -= w;
-            for (int row = j + 1 + qg; row < K; row += gq) G[c][row] -= w * G[j][row];
-          }
-        }
-      __syncthreads();
-    }
-    if constexpr (!VG) {
-      // Q = H_0 H_1 ... H_{K-1} formed in the right-vector array (identity so
-      // far), from the reflectors kept below G's diagonal, last one first: the
-      // rotations then carry Q along, so the array ends as Q V_x, the left
-      // vectors, with no back-transform (and no LDS for the reflectors)
-      for (int j = K - 1; j >= 0; --j) {
-        const T tau = tauq[j];
-        if (tau != T(0))
-          for (int c0 = j; c0 < K; c0 += NT / gq) {
-            const int c = c0 + qc;
-            T w = T(0);
-            if (c < K) {
-              if (qg == 0) w = VA(c, j);
-              for (int row = j + 1 + qg; row < K; row += gq) w += G[j][row] * VA(c, row);
-            }
-            w = group_sum(w, gq) * tau;
-            if (c < K) {
-              if (qg == 0) VA(c, j) -= w;
-              for (int row = j + 1 + qg; row < K; row += gq) VA(c, row) -= w * G[j][row];
-            }
-          }
-        __syncthreads();
-      }
-    }
-    // G = R^T (in place): column j of G becomes row j of R, and the reflectors
-    // below R's diagonal give way to zeros
-    for (int e = tid; e < K * K; e += NT) {
-      const int c = e / K, row = e % K;
-      if (row > c) {
-        G[c][row] = G[row][c];
-        G[row][c] = T(0);
-      }
-    }
-    __syncthreads();
-  }
-  for (int j = tid; j < K; j += NT) {
-    T c2 = T(0);
-    for (int row = 0; row < K; ++row) c2 += G[j][row] * G[j][row];
-    sig[j] = c2;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    T fro2 = T(0);
-    for (int j = 0; j < K; ++j) fro2 += sig[j];
-    // columns below u ||M||_F (u the unit roundoff) are numerically zero: rotating
-    // them only churns rounding noise.  The floor also stays a factor 16 under the
-    // truncation threshold eps ||sigma|| / sqrt(K) of an eps-rank decision, so in
-    // FP32 at eps near 1e-6 the columns the rank is decided on are still rotated.
-    T fl = Eps<T>::v;
-    if (it.fixed_rank < 0 && it.eps > 0.0) fl = fmin(fl, static_cast<T>(it.eps / (16.0 * sqrt((double)K))));
-    tiny_sh = fl * fl * fro2;
-  }
-  __syncthreads();
-  const T tiny = tiny_sh;
-  const int K2 = K + (K & 1);
-  const int P = K2 / 2;
-  int gl = 64;
-  while (gl > 1 && P * gl > NT) gl >>= 1;
-  const int p = tid / gl, sub = tid % gl;
-  // rotation threshold: above the rounding noise of a length-K dot product
-  const T tol = T(8 * max(K, 8)) * Eps<T>::v;
-  const T itol = T(1) / tol;
-  // The rounds run the round-robin schedule cyclically and stop once K2 - 1
-  // consecutive rounds (every pair once, from any starting round) rotated
-  // nothing: then no column changed while every pair was tested, as after a
-  // rotation-free sweep.
-  int rounds = 0;
-  if (K >= 2) {
-    int quiet = 0;
-    for (int r = 0; quiet < K2 - 1 && rounds < 60 * (K2 - 1); r = (r + 1 == K2 - 1) ? 0 : r + 1) {
-      ++rounds;
-      int rotated = 0;
-      if (p < P) {
-        int i = rr_pos(p, r, K2), j = rr_pos(K2 - 1 - p, r, K2);
-        if (i > j) {
-          const int tmp = i;
-          i = j;
-          j = tmp;
-        }
-        if (j < K) {
-          T al = T(0), be = T(0), ga = T(0);
-          for (int row = sub; row < K; row += gl) {
-            const T x = G[i][row], y = G[j][row];
-            al += x * x;
-            be += y * y;
-            ga += x * y;
-          }
-          al = group_sum(al, gl);
-          be = group_sum(be, gl);
-          ga = group_sum(ga, gl);
-          const T gt = ga * itol;  // |ga| > tol sqrt(al be), squared with no underflow (al, be > tiny)
-          if (al > tiny && be > tiny && gt * gt > al * be) {
-            T cth, sth;
-            jacobi_rotation(al, be, ga, cth, sth);
-            for (int row = sub; row < K; row += gl) {
-              const T x = G[i][row], y = G[j][row];
-              G[i][row] = cth * x - sth * y;
-              G[j][row] = sth * x + cth * y;
-              if constexpr (!VG) {
-                const T vx = VA(i, row), vy = VA(j, row);
-                VA(i, row) = cth * vx - sth * vy;
-                VA(j, row) = sth * vx + cth * vy;
-              }
-            }
-            rotated = 1;
-          }
-        }
-      }
-      quiet = __syncthreads_or(rotated) ? 0 : quiet + 1;
-    }
-  }
-  const int sweeps = (rounds + K2 - 2) / max(1, K2 - 1);
-  if (tid == 0 && it.stats != nullptr) {
-    // this workgroup's copy of the counters (a line of its own: no contention
-    // between the items of a launch)
-    int32_t* st = it.stats + (blockIdx.x % kCounterCopies) * kCounterStride;
-    atomicAdd(st, 1);
-    atomicAdd(st + 1, sweeps);
-    atomicMax(st + 2, sweeps);
-  }
-  for (int j = tid; j < K; j += NT) {
-    T s = T(0);
-    for (int row = 0; row < K; ++row) s += G[j][row] * G[j][row];
-    sig[j] = sqrt(s);
-  }
-  __syncthreads();
-  for (int j = tid; j < K; j += NT) {
-    int rk = 0;
-    const T sj = sig[j];
-    for (int i = 0; i < K; ++i)
-      if (sig[i] > sj || (sig[i] == sj && i < j)) ++rk;
-    order[rk] = j;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int r;
-    if (it.fixed_rank >= 0) {
-      r = min(it.fixed_rank, K);
-    } else {
-      const int md = (it.kdim > 0) ? min(it.kdim, K) : K;
-      T ss = T(0);
-      for (int i = 0; i < md; ++i) {
-        const T v = sig[order[i]];
-        ss += v * v;
-      }
-      const T threshold = static_cast<T>(it.eps) * sqrt(ss);
-      r = 0;
-      T err;
-      do {
-        ++r;
-        err = T(0);
-        if (r < md) {
-          const T sr = sig[order[r]];
-          for (int jj = r; jj < md; ++jj) err += sr * sr;
-        }
-      } while (r < md && sqrt(err) > threshold);
-    }
-    if (r > it.cap) {
-      if (it.rank_out) *it.rank_out = it.cap_trunc ? it.cap : -r;
-      r = it.cap;
-    } else if (it.rank_out) {
-      *it.rank_out = r;
-    }
-    rank_sh = r;
-  }
-  __syncthreads();
-  const int r = rank_sh;
-  // normalise left vectors in place
-  for (int e = tid; e < K * K; e += NT) {
-    const int c = e / K, row = e % K;
-    const T s = sig[c];
-    if (s > T(0)) G[c][row] = G[c][row] / s;
-  }
-  __syncthreads();
-  // Orthonormal completion of kept left vectors whose singular value is
-  // numerically zero (below eps * ||M||_F: Jacobi leaves those columns
-  // unrotated): two passes of classical Gram-Schmidt of e_u against the
-  // earlier kept vectors, accepted when the remainder keeps norm^2 > thr.
-  // Candidates are scanned from u = K - 1 down (the pivoted leading coordinates
-  // carry the kept vectors) and the scan resumes where the previous column's
-  // stopped: a rejected remainder only shrinks as the span grows, and an
-  // accepted e_u lies in it.  The remainders' squared norms sum to K - c, so a
-  // second scan with thr = 1/(4K) always accepts one.
-  const T sig_floor = sqrt(tiny);
-  int u = K - 1;
-  T thr = T(0.25);
-  for (int c = 0; c < r; ++c) {
-    const int src = order[c];
-    if (sig[src] > sig_floor) continue;
-    for (int tries = 0; tries < 2 * K; ++tries, --u) {
-      if (u < 0) {
-        u = K - 1;
-        thr = T(0.25) / T(K);
-      }
-      for (int row = tid; row < K; row += NT) G[src][row] = (row == u) ? T(1) : T(0);
-      __syncthreads();
-      for (int pass = 0; pass < 2; ++pass) {
-        for (int pp = tid; pp < c; pp += NT) {
-          const int ps = order[pp];
-          T d = T(0);
-          for (int row = 0; row < K; ++row) d += G[ps][row] * G[src][row];
-          coef[pp] = d;
-        }
-        __syncthreads();
-        for (int row = tid; row < K; row += NT) {
-          T x = G[src][row];
-          for (int pp = 0; pp < c; ++pp) x -= coef[pp] * G[order[pp]][row];
-          G[src][row] = x;
-        }
-        __syncthreads();
-      }
-      if (tid == 0) {
-        T nn = T(0);
-        for (int row = 0; row < K; ++row) nn += G[src][row] * G[src][row];
-        accept_sh = nn > thr;
-        coef[0] = (nn > T(0)) ? T(1) / sqrt(nn) : T(0);
-      }
-      __syncthreads();
-      const int ok = accept_sh;
-      const T inv = coef[0];
-      __syncthreads();
-      if (ok) {
-        for (int row = tid; row < K; row += NT) G[src][row] *= inv;
-        __syncthreads();
-        --u;
-        break;
-      }
-    }
-  }
-  T* S = static_cast<T*>(it.S);
-  T* Um = static_cast<T*>(it.Um);
-  T* Vm = static_cast<T*>(it.Vm);
-  if (S != nullptr)
-    for (int e = tid; e < r * r; e += NT) {
-      const int i = e / r, j = e % r;
-      S[i * it.lds + j] = (i == j) ? sig[order[i]] * unscale : T(0);
-    }
-  if constexpr (PRE) {
-    // M = (Q V_x) Sigma (P U_x)^T: right vectors from G (rows permuted back),
-    // left vectors Q V_x (the rotated Q), or, in VG mode, M v / sigma
-    for (int e = tid; e < K * r; e += NT) {
-      const int row = e / r, c = e % r;
-      if (Vm != nullptr) Vm[perm[row] * it.ldv + c] = G[order[c]][row];
-    }
-    if constexpr (!VG) {
-      for (int e = tid; e < K * r; e += NT) {
-        const int row = e / r, c = e % r;
-        if (Um != nullptr) Um[row * it.ldu + c] = VA(order[c], row);
-      }
-    } else if (Um != nullptr) {
-      // u_c = M P g_c / sigma_c: column perm[j] of M against entry j of g_c, a wave per output
-      const int lane = tid & 63, wv = tid >> 6;
-      for (int o = wv; o < K * r; o += NT / 64) {
-        const int row = o / r, c = o % r;
-        const int src = order[c];
-        const T sc = sig[src];
-        T acc = T(0);
-        for (int j2 = lane; j2 < K; j2 += 64) acc += vg[(int64_t)perm[j2] * K + row] * G[src][j2];
-        acc = wave_sum(acc);
-        if (lane == 0) Um[row * it.ldu + c] = (sc > sig_floor) ? acc / sc : T(0);
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Register-resident one-sided Jacobi SVD for K <= KMAX (16 or 32): one wave per
-// core and no LDS traffic inside the rounds.  The round-robin schedule has K2
-// positions (K rounded up to even; a zero column pads odd K) in NS slots of two:
-// the top of slot s is position s, its bottom position K2-1-s.  Lane l serves
-// slot s = l % NS together with the other NL lanes of that slot, holding rows
-// g + NL q (g = l / NS) of the top column in x[], of the bottom column in y[] and
-// of their right vectors in vx[], vy[].  A round rotates every slot's pair at
-// once; the columns then move one place round the circle (top 0 fixed, top k-1
-// -> top k, bottom 0 -> top 1, bottom k+1 -> bottom k, top P-1 -> bottom P-1).
-// Neighbouring slots are neighbouring lanes, so a move is one DPP wave shift per
-// register; the column sums are a DPP / swizzle / permlane butterfly.
-// ---------------------------------------------------------------------------
-// (lane 0, resp. 63, receives zero: bound_ctrl writes every lane, so no old value is needed)
-template <int CTRL>
-__device__ __forceinline__ int dpp_bound_i(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
-}
-__device__ __forceinline__ float wave_shr1(float v) {  // lane l receives lane l - 1
-  return __int_as_float(dpp_bound_i<0x138>(__float_as_int(v)));
-}
-__device__ __forceinline__ double wave_shr1(double v) {
-  return __hiloint2double(dpp_bound_i<0x138>(__double2hiint(v)), dpp_bound_i<0x138>(__double2loint(v)));
-}
-__device__ __forceinline__ float wave_shl1(float v) {  // lane l receives lane l + 1
-  return __int_as_float(dpp_bound_i<0x130>(__float_as_int(v)));
-}
-__device__ __forceinline__ double wave_shl1(double v) {
-  return __hiloint2double(dpp_bound_i<0x130>(__double2hiint(v)), dpp_bound_i<0x130>(__double2loint(v)));
-}
 __device__ __forceinline__ float half_max(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
   return fmaxf(__int_as_float(r[0]), __int_as_float(r[1]));
@@ -2273,374 +1762,644 @@ __device__ __forceinline__ T wave_max(T v) {
   v = fmax(v, xor16(v));
   return half_max(v);
 }
-// v[l] + v[l ^ 16] through v_permlane16_swap (gfx950), operands in the same order in every lane
-__device__ __forceinline__ float pair16_sum(float v) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
-  return __int_as_float(r[0]) + __int_as_float(r[1]);
+// ---------------------------------------------------------------------------
+// LDS Jacobi SVD for K <= KMAX, one workgroup of KMAX / 2 groups of GL lanes per
+// core: group g serves columns g and g + KMAX / 2 (QR phase), or the column pair
+// of its slot (rotations).  A lane holds rows VW sub + VW GL t + e, so a group
+// reads a column as contiguous 16-byte words: no bank conflicts.
+//   1. M is formed in registers and scaled by a power of two (max |M_ij| in
+//      [1, 2): exact, and squared norms stay clear of underflow).
+//   2. Column-pivoted Householder QR, M P = Q R, in registers: every wave offers
+//      its best remaining column through LDS, so a step costs one barrier.  It
+//      stops once the trailing block is below delta = max(u, 1e-3 eps) ||M||_F
+//      (u: the unit roundoff, eps: the truncation accuracy): the block enters the
+//      kept singular values in second order only (sigma^2 moves by at most
+//      delta^2), and the rotations then run on rp < K columns.
+//   3. One-sided Jacobi on R^T (K x rp), whose graded rows converge in few sweeps
+//      (Drmac-Veselic), a round-robin schedule, one barrier a round.  The
+//      rotations also turn Q into the left vectors.  VG (FP64, K > 64: the second
+//      array does not fit LDS): the left vectors are formed afterwards as
+//      M v / sigma by FP64 MFMA from a copy of M in global scratch.
+// Bound: latency of the dependent steps of one core (QR steps and rounds, about
+// 0.45 us a round at K = 16 to 0.9 us at K = 64 in FP64); in large batches the LDS
+// traffic of the rotations.  Launch averages, before (one array read with scalar
+// strided columns, norms recomputed per QR step, a serial pivot search, K full
+// columns; a register kernel for K <= 16 and FP64 K <= 32) -> now: FP64 K <= 16,
+// 778 cores 69 -> 35 us; FP64 K <= 32, 590 cores 214 -> 52 us; FP64 K <= 64, 165
+// cores 1.78 -> 0.69 ms; FP64 K <= 128, 5 cores 2.84 -> 0.95 ms; FP32 K <= 16, 672
+// cores 22.6 -> 18.5 us; FP32 K <= 64, 1231 cores 1.29 -> 0.51 ms; FP32 K <= 128,
+// 817 cores 5.66 -> 1.45 ms.
+// ---------------------------------------------------------------------------
+template <typename T, int N>
+struct LdsVec {
+  typedef T type __attribute__((ext_vector_type(N)));
+};
+// 1 / sqrt(x): the FP64 hardware estimate with one third-order correction (the
+// estimate's relative error, below 1e-7, enters cubed)
+__device__ __forceinline__ double rsqrt_nr(double x) {
+  const double r = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * r, r, 1.0);
+  return fma(r * e, fma(0.375, e, 0.5), r);
 }
-__device__ __forceinline__ double pair16_sum(double v) {
-  const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
-  const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
-  return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+__device__ __forceinline__ double sqrt_nr(double x) { return x > 0.0 ? x * rsqrt_nr(x) : x; }
+__device__ __forceinline__ float sqrt_nr(float x) { return sqrtf(x); }
+__device__ __forceinline__ double inv_nr(double x) { return d64::rcp2(x); }
+__device__ __forceinline__ float inv_nr(float x) { return 1.0f / x; }
+// Rotation (c, s) that zeroes the off-diagonal of [[al, ga], [ga, be]].  FP64:
+// cos 2t = |d| / h and sin 2t = 2 ga / h with d = be - al, h = sqrt(d^2 + 4 ga^2):
+// two reciprocal square roots, no division (the squares cannot underflow, since
+// al and be exceed (u ||M||_F)^2 after the scaling).  FP32, whose squares could:
+// Rutishauser's formulas, t = sign(zeta) / (|zeta| + sqrt(1 + zeta^2)), zeta =
+// (be - al) / (2 ga), c = 1 / sqrt(1 + t^2), s = c t, on the hardware reciprocal
+// and roots (about 1 ulp: only the angle moves, the rotation stays orthogonal).
+__device__ __forceinline__ void jacobi_rotation(double al, double be, double ga, double& c, double& s) {
+  const double d = be - al;
+  const double w = rsqrt_nr(fma(d, d, 4.0 * ga * ga));
+  const double c2 = fma(0.5 * fabs(d), w, 0.5);
+  const double rc = rsqrt_nr(c2);
+  c = c2 * rc;
+  s = copysign(ga * w * rc, d >= 0.0 ? ga : -ga);
 }
-// sum over the NL lanes of a slot (lanes s + NS t), the same bits in each of them
-template <int NL, typename T>
-__device__ __forceinline__ T slot_sum(T v) {
-  static_assert(NL == 4 || NL == 8, "slot of 4 or 8 lanes");
-  if constexpr (NL == 8) v += dpp_mov<0x128>(v);  // row_ror:8 = lane l ^ 8
-  return half_sum(pair16_sum(v));
+__device__ __forceinline__ void jacobi_rotation(float al, float be, float ga, float& c, float& s) {
+  const float zeta = (be - al) * __builtin_amdgcn_rcpf(2.0f * ga);
+  const float t = copysignf(1.0f, zeta) * __builtin_amdgcn_rcpf(fabsf(zeta) + __builtin_amdgcn_sqrtf(1.0f + zeta * zeta));
+  c = __builtin_amdgcn_rsqf(1.0f + t * t);
+  s = c * t;
+}
+__device__ __forceinline__ unsigned umax32(unsigned a, unsigned b) { return a > b ? a : b; }
+// max over the 64 / GL groups of a wave of a value uniform over each group
+template <int GL>
+__device__ __forceinline__ unsigned groups_umax(unsigned k) {
+  if constexpr (GL == 8) k = umax32(k, (unsigned)dpp_i<0x128>((int)k));
+  k = umax32(k, (unsigned)swz16_i((int)k));
+  const auto r = __builtin_amdgcn_permlane32_swap((int)k, (int)k, false, false);
+  return umax32((unsigned)r[0], (unsigned)r[1]);
+}
+// max over NW <= 16 values, lane l holding value l % NW
+template <int NW>
+__device__ __forceinline__ unsigned lanes_umax(unsigned k) {
+  if constexpr (NW > 1) k = umax32(k, (unsigned)dpp_i<0xB1>((int)k));
+  if constexpr (NW > 2) k = umax32(k, (unsigned)dpp_i<0x4E>((int)k));
+  if constexpr (NW > 4) k = umax32(k, (unsigned)dpp_i<0x141>((int)k));
+  if constexpr (NW > 8) k = umax32(k, (unsigned)dpp_i<0x140>((int)k));
+  return k;
+}
+template <int GL>
+__device__ __forceinline__ int group_isum(int v) {
+  v += dpp_i<0xB1>(v);
+  v += dpp_i<0x4E>(v);
+  v += dpp_i<0x141>(v);
+  if constexpr (GL == 16) v += dpp_i<0x140>(v);
+  return v;
 }
 
-template <typename T, int KMAX, class Src>
-__global__ __launch_bounds__(64) void svd_reg_kernel(Src items) {
-  constexpr int NS = KMAX / 2, NL = 64 / NS, NR = KMAX / NL;
+// sum_e x[e] y[e] as a tree over pairs: a shorter dependent chain than one running
+// sum, and in FP32 a smaller rounding error
+template <int N, typename T>
+__device__ __forceinline__ T dot_tree(const T (&x)[N], const T (&y)[N]) {
+  constexpr int H = (N + 1) / 2;
+  T p[H];
+#pragma unroll
+  for (int k = 0; k < H; ++k) {
+    p[k] = x[2 * k] * y[2 * k];
+    if (2 * k + 1 < N) p[k] += x[2 * k + 1] * y[2 * k + 1];
+  }
+#pragma unroll
+  for (int s = 1; s < H; s *= 2)
+#pragma unroll
+    for (int k = 0; k + s < H; k += 2 * s) p[k] += p[k + s];
+  return p[0];
+}
+
+template <typename T, int KMAX, int GL, bool VG, class Src>
+__global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
+  constexpr int NG = KMAX / 2, NT = NG * GL, NW = NT / 64, RL = KMAX / GL;
+  constexpr int VW = (sizeof(T) == 4 && RL % 4 == 0) ? 4 : 2, NC = RL / VW;
+  constexpr int LD = KMAX + VW;
+  static_assert(GL == 8 || GL == 16, "groups of 8 or 16 lanes");
+  static_assert(KMAX <= 128 && NT % 64 == 0 && 2 * NW <= KMAX && RL % VW == 0, "shape");
+  using vec = typename LdsVec<T, VW>::type;
   const SvdItem it = items.get(blockIdx.x);
   const int K = it.K;
-  const int lane = threadIdx.x;
-  const int s = lane % NS, g = lane / NS;
-  // staging (Ru, or M in mode 0; Rv); the left vectors on the completion path
-  __shared__ T A1[KMAX][KMAX + 1];
-  __shared__ T A2[KMAX][KMAX + 1];
-  __shared__ T sig[KMAX];   // by position
-  __shared__ T sigs[KMAX];  // descending
+  __shared__ __align__(16) T G[KMAX * LD];
+  __shared__ __align__(16) T Vs[VG ? VW : KMAX * LD];  // reflectors, then Q, then the left vectors
+  __shared__ T taus[KMAX], sig[KMAX], sigs[KMAX], coef[KMAX];
+  __shared__ T candq[2][NW], wmax[NW];
+  __shared__ unsigned candk[2][NW];
   __shared__ int order[KMAX];
-  __shared__ int rk_of[KMAX];
-  __shared__ T coef[KMAX];
+  __shared__ int rank_sh, lastrot_sh, accept_sh;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int g = tid / GL, sub = tid % GL;
+  T* vg = static_cast<T*>(it.vwork);
   if (K <= 0) {
-    if (lane == 0 && it.rank_out) *it.rank_out = 0;
+    if (tid == 0 && it.rank_out) *it.rank_out = 0;
     return;
   }
-  const int K2 = K + (K & 1), P = K2 / 2;
-  const int pt = s, pb = K2 - 1 - s;
-  const bool act = s < P;
+  if constexpr (VG) {
+    if (vg == nullptr) {  // missing scratch: report an impossible rank instead of touching memory
+      if (tid == 0 && it.rank_out) *it.rank_out = -(1 << 20);
+      return;
+    }
+  }
+  const int c0 = g, c1 = g + NG;
+  auto row_of = [&](int e) { return VW * sub + VW * GL * (e / VW) + (e % VW); };
+  auto load_col = [&](const T* col, T (&v)[RL]) {
+#pragma unroll
+    for (int t = 0; t < NC; ++t) {
+      const vec w = *reinterpret_cast<const vec*>(col + VW * sub + VW * GL * t);
+#pragma unroll
+      for (int e = 0; e < VW; ++e) v[VW * t + e] = w[e];
+    }
+  };
+  auto store_col = [&](T* col, const T (&v)[RL]) {
+#pragma unroll
+    for (int t = 0; t < NC; ++t) {
+      vec w;
+#pragma unroll
+      for (int e = 0; e < VW; ++e) w[e] = v[VW * t + e];
+      *reinterpret_cast<vec*>(col + VW * sub + VW * GL * t) = w;
+    }
+  };
+  // ---- 1. the core, columns c0 and c1 in registers ---------------------------
+  T x0[RL], x1[RL];
+#pragma unroll
+  for (int e = 0; e < RL; ++e) x0[e] = x1[e] = T(0);
   if (it.mode == 0) {
     const T* M = static_cast<const T*>(it.M);
 #pragma unroll
-    for (int k = 0; k < KMAX * KMAX / 64; ++k) {
-      const int e = lane + 64 * k;
-      const int i = e / KMAX, j = e % KMAX;
-      A1[i][j] = (i < K && j < K) ? M[i * it.m_rs + j * it.m_cs] : T(0);
+    for (int e = 0; e < RL; ++e) {
+      const int row = row_of(e);
+      if (row < K && c0 < K) x0[e] = M[row * it.m_rs + c0 * it.m_cs];
+      if (row < K && c1 < K) x1[e] = M[row * it.m_rs + c1 * it.m_cs];
     }
   } else {
+    // M(i, j) = sum_t Ru(i, t) Rv(j, t): Ru (and Rv when there is room) staged by
+    // columns; Ru and Rv are upper triangular below their first ka rows
     const int J = it.kx;
     const T* Ru = static_cast<const T*>(it.Ru);
     const T* Rv = static_cast<const T*>(it.Rv);
-#pragma unroll
-    for (int k = 0; k < KMAX * KMAX / 64; ++k) {
-      const int e = lane + 64 * k;
-      const int i = e / KMAX, t = e % KMAX;
-      const bool in = i < K && t < J;
-      A1[i][t] = in ? Ru[i * it.ldr + t] : T(0);
-      A2[i][t] = in ? Rv[i * it.ldr + t] : T(0);
+    for (int e = tid; e < KMAX * J; e += NT) {
+      const int i = e / J, t = e - (e / J) * J;
+      G[t * LD + i] = (i < K) ? Ru[i * it.ldr + t] : T(0);
+      if constexpr (!VG) Vs[t * LD + i] = (i < K) ? Rv[i * it.ldr + t] : T(0);
     }
-  }
-  __syncthreads();
-  T x[NR], y[NR], vx[NR], vy[NR];
+    T rv0[VG ? KMAX / GL : 1], rv1[VG ? KMAX / GL : 1];
+    if constexpr (VG) {
 #pragma unroll
-  for (int q = 0; q < NR; ++q) {
-    const int ri = g + NL * q;
-    x[q] = T(0);
-    y[q] = T(0);
-    vx[q] = (act && ri == pt && ri < K) ? T(1) : T(0);
-    vy[q] = (act && ri == pb && ri < K) ? T(1) : T(0);
-  }
-  if (act) {
-    if (it.mode == 0) {
-#pragma unroll
-      for (int q = 0; q < NR; ++q) {
-        x[q] = A1[g + NL * q][pt];
-        y[q] = A1[g + NL * q][pb];
+      for (int k = 0; k < KMAX / GL; ++k) {
+        const int t = sub + GL * k;
+        rv0[k] = (t < J && c0 < K) ? Rv[c0 * it.ldr + t] : T(0);
+        rv1[k] = (t < J && c1 < K) ? Rv[c1 * it.ldr + t] : T(0);
       }
+    }
+    __syncthreads();
+    auto accum = [&](int t, T a, T b) {
+      T u[RL];
+      load_col(G + t * LD, u);
+#pragma unroll
+      for (int e = 0; e < RL; ++e) {
+        x0[e] += u[e] * a;
+        x1[e] += u[e] * b;
+      }
+    };
+    if constexpr (VG) {
+#pragma unroll
+      for (int k = 0; k < KMAX / GL; ++k)
+        for (int s = 0; s < GL; ++s) {
+          const int t = GL * k + s;
+          const T a = __shfl(rv0[k], s, GL), b = __shfl(rv1[k], s, GL);
+          if (t < J) accum(t, a, b);
+        }
     } else {
-      // M(i, j) = sum_t Ru(i, t) Rv(j, t) (+ Sa(i, j) inside the leading ka x ka block)
-      const int J = it.kx;
-      for (int t = 0; t < J; ++t) {
-        const T a = A2[pt][t], b = A2[pb][t];
+      for (int t = max(0, c0 - it.ka); t < J; ++t) accum(t, Vs[t * LD + c0], Vs[t * LD + c1]);
+    }
+    if (it.ka > 0) {
+      const T* Sa = static_cast<const T*>(it.Sa);
 #pragma unroll
-        for (int q = 0; q < NR; ++q) {
-          const T u = A1[g + NL * q][t];
-          x[q] += u * a;
-          y[q] += u * b;
-        }
-      }
-      if (it.ka > 0) {
-        const T* Sa = static_cast<const T*>(it.Sa);
-#pragma unroll
-        for (int q = 0; q < NR; ++q) {
-          const int ri = g + NL * q;
-          if (ri < it.ka) {
-            if (pt < it.ka) x[q] += Sa[ri * it.lds_in + pt];
-            if (pb < it.ka) y[q] += Sa[ri * it.lds_in + pb];
-          }
-        }
+      for (int e = 0; e < RL; ++e) {
+        const int row = row_of(e);
+        if (row < it.ka && c0 < it.ka) x0[e] += Sa[row * it.lds_in + c0];
+        if (row < it.ka && c1 < it.ka) x1[e] += Sa[row * it.lds_in + c1];
       }
     }
   }
-  // exact power-of-two scaling: max |M_ij| in [1, 2)
   T mx = T(0);
 #pragma unroll
-  for (int q = 0; q < NR; ++q) mx = fmax(mx, fmax(fabs(x[q]), fabs(y[q])));
-  const T amax = wave_max(mx);
+  for (int e = 0; e < RL; ++e) mx = fmax(mx, fmax(fabs(x0[e]), fabs(x1[e])));
+  mx = wave_max(mx);
+  if (lane == 0) wmax[wv] = mx;
+  __syncthreads();
+  T amax = wmax[0];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) amax = fmax(amax, wmax[w]);
   int sexp = 0;
   if (amax > T(0) && isfinite(amax)) sexp = ilogb(amax);
   const T scale = ldexp(T(1), -sexp), unscale = ldexp(T(1), sexp);
-  T f2 = T(0);
 #pragma unroll
-  for (int q = 0; q < NR; ++q) {
-    x[q] *= scale;
-    y[q] *= scale;
-    f2 += x[q] * x[q] + y[q] * y[q];
+  for (int e = 0; e < RL; ++e) {
+    x0[e] *= scale;
+    x1[e] *= scale;
   }
-  const T fro2 = wave_sum(f2);
-  // numerically zero columns (below u ||M||_F, and 16x under an eps-rank
-  // threshold) are not rotated
-  T fl = Eps<T>::v;
-  if (it.fixed_rank < 0 && it.eps > 0.0) fl = fmin(fl, static_cast<T>(it.eps / (16.0 * sqrt((double)K))));
-  const T tiny = fl * fl * fro2;
-  const T tol = T(8 * max(K, 8)) * Eps<T>::v;
-  const T itol = T(1) / tol;
-  // cyclic rounds until K2 - 1 consecutive rounds rotate nothing
-  int rounds = 0;
-  if (K >= 2) {
-    int quiet = 0;
-    while (quiet < K2 - 1 && rounds < 60 * (K2 - 1)) {
-      ++rounds;
-      T al = T(0), be = T(0), ga = T(0);
+  T q0 = group_sum(dot_tree(x0, x0), GL), q1 = group_sum(dot_tree(x1, x1), GL);
+  if (sub == 0) {
+    sig[c0] = q0;
+    sig[c1] = q1;
+  }
+  if constexpr (VG) {
+    // the scaled core, column j at vg + j K
 #pragma unroll
-      for (int q = 0; q < NR; ++q) {
-        al += x[q] * x[q];
-        be += y[q] * y[q];
-        ga += x[q] * y[q];
-      }
-      al = slot_sum<NL>(al);
-      be = slot_sum<NL>(be);
-      ga = slot_sum<NL>(ga);
-      const T gt = ga * itol;
-      const bool rot = act && al > tiny && be > tiny && gt * gt > al * be;
-      if (rot) {
-        T cth, sth;
-        jacobi_rotation(al, be, ga, cth, sth);
-#pragma unroll
-        for (int q = 0; q < NR; ++q) {
-          const T a = x[q], b = y[q];
-          x[q] = cth * a - sth * b;
-          y[q] = sth * a + cth * b;
-          const T va = vx[q], vb = vy[q];
-          vx[q] = cth * va - sth * vb;
-          vy[q] = sth * va + cth * vb;
-        }
-      }
-      quiet = __any(rot) ? 0 : quiet + 1;
-      if (P > 1) {
-#pragma unroll
-        for (int q = 0; q < NR; ++q) {
-          const T nt = wave_shr1((s == 0) ? y[q] : x[q]);
-          const T ntv = wave_shr1((s == 0) ? vy[q] : vx[q]);
-          const T nb = wave_shl1(y[q]);
-          const T nbv = wave_shl1(vy[q]);
-          if (s == P - 1) {
-            y[q] = x[q];
-            vy[q] = vx[q];
-          } else {
-            y[q] = nb;
-            vy[q] = nbv;
-          }
-          if (s != 0) {
-            x[q] = nt;
-            vx[q] = ntv;
-          }
-        }
-      }
+    for (int e = 0; e < RL; ++e) {
+      const int row = row_of(e);
+      if (row < K && c0 < K) vg[(int64_t)c0 * K + row] = x0[e];
+      if (row < K && c1 < K) vg[(int64_t)c1 * K + row] = x1[e];
     }
   }
-  const int sweeps = (rounds + K2 - 2) / max(1, K2 - 1);
-  if (lane == 0 && it.stats != nullptr) {
+  if (tid == 0) lastrot_sh = 0;
+  __syncthreads();
+  T fro2 = T(0);
+#pragma unroll
+  for (int k = 0; k < (KMAX + 63) / 64; ++k)
+    if (lane + 64 * k < KMAX) fro2 += sig[lane + 64 * k];
+  fro2 = wave_sum(fro2);
+  // columns below u ||M||_F are numerically zero: rotating them only churns
+  // rounding noise.  The floor also stays a factor 16 under the truncation
+  // threshold eps ||sigma|| / sqrt(K) of an eps-rank decision, so in FP32 at eps
+  // near 1e-6 the columns the rank is decided on are still rotated.
+  T fl = Eps<T>::v, fd = Eps<T>::v;
+  if (it.fixed_rank < 0 && it.eps > 0.0) {
+    fl = fmin(fl, static_cast<T>(it.eps / (16.0 * sqrt((double)K))));
+    fd = fmax(fl, static_cast<T>(1e-3 * it.eps));
+  }
+  const T tiny = fl * fl * fro2, delta2 = fd * fd * fro2;
+  // ---- 2. pivoted QR, columns in registers -----------------------------------
+  bool live0 = c0 < K, live1 = c1 < K;
+  int rp = 0;
+  for (; rp < K; ++rp) {
+    const int buf = rp & 1;
+    // the remaining column of largest norm: the norm's leading float bits above
+    // the column index (the smaller index on a tie)
+    const unsigned k0 = live0 ? ((__float_as_uint((float)q0) & ~0x7Fu) | (unsigned)(127 - c0)) : 0u;
+    const unsigned k1 = live1 ? ((__float_as_uint((float)q1) & ~0x7Fu) | (unsigned)(127 - c1)) : 0u;
+    const unsigned kg = umax32(k0, k1), kw = groups_umax<GL>(kg);
+    if (kg == kw && (live0 || live1)) {
+      const bool first = k0 == kw && live0;
+      T xs[RL];
+#pragma unroll
+      for (int e = 0; e < RL; ++e) xs[e] = first ? x0[e] : x1[e];
+      store_col(G + (buf * NW + wv) * LD, xs);
+      if (sub == 0) candq[buf][wv] = first ? q0 : q1;
+    }
+    if (lane == 0) candk[buf][wv] = kw;
+    __syncthreads();
+    const unsigned ka = lanes_umax<NW>(candk[buf][lane % NW]);
+    const int pv = 127 - (int)(ka & 0x7Fu);
+    const int pw = ((pv >= NG ? pv - NG : pv) * GL) >> 6;
+    const T q = candq[buf][pw];
+    if (q * T(K - rp) <= delta2) break;
+    const T* pc = G + (buf * NW + pw) * LD;
+    T v[RL];
+    load_col(pc, v);
+    const T alpha = pc[rp];
+    const T nrm = sqrt_nr(q);
+    const T beta = (alpha >= T(0)) ? -nrm : nrm;
+    const T tau = inv_nr(q - alpha * beta);  // H = I - tau w w^T, w = x - beta e
+#pragma unroll
+    for (int e = 0; e < RL; ++e) {
+      const int row = row_of(e);
+      v[e] = (row > rp) ? v[e] : (row == rp ? alpha - beta : T(0));
+    }
+    if constexpr (!VG) {
+      if (g == rp % NG) {
+        store_col(Vs + rp * LD, v);
+        if (sub == 0) taus[rp] = tau;
+      }
+    }
+    live0 = live0 && c0 != pv;
+    live1 = live1 && c1 != pv;
+    // (a column reduced before is zero below its diagonal: its product vanishes)
+    const T d0 = group_sum(dot_tree(v, x0), GL) * tau, d1 = group_sum(dot_tree(v, x1), GL) * tau;
+    T z0[RL], z1[RL];
+#pragma unroll
+    for (int e = 0; e < RL; ++e) {
+      const int row = row_of(e);
+      x0[e] -= d0 * v[e];
+      x1[e] -= d1 * v[e];
+      if (c0 == pv) x0[e] = (row > rp) ? T(0) : (row == rp ? beta : x0[e]);
+      if (c1 == pv) x1[e] = (row > rp) ? T(0) : (row == rp ? beta : x1[e]);
+      z0[e] = (row > rp) ? x0[e] : T(0);
+      z1[e] = (row > rp) ? x1[e] : T(0);
+    }
+    q0 = group_sum(dot_tree(z0, z0), GL);
+    q1 = group_sum(dot_tree(z1, z1), GL);
+  }
+  const int n = rp;
+  __syncthreads();  // the last candidates are read, the reflectors complete
+  if constexpr (!VG) {
+    // Q e_c for c = c0, c1 (every column: the ones past n complete the left basis)
+    T y0[RL], y1[RL];
+#pragma unroll
+    for (int e = 0; e < RL; ++e) {
+      y0[e] = (row_of(e) == c0) ? T(1) : T(0);
+      y1[e] = (row_of(e) == c1) ? T(1) : T(0);
+    }
+    for (int j = n - 1; j >= 0; --j) {
+      T v[RL];
+      load_col(Vs + j * LD, v);
+      const T tau = taus[j];
+      const T d0 = group_sum(dot_tree(v, y0), GL) * tau, d1 = group_sum(dot_tree(v, y1), GL) * tau;
+#pragma unroll
+      for (int e = 0; e < RL; ++e) {
+        y0[e] -= d0 * v[e];
+        y1[e] -= d1 * v[e];
+      }
+    }
+    __syncthreads();
+    store_col(Vs + c0 * LD, y0);
+    store_col(Vs + c1 * LD, y1);
+  }
+  // G = R^T: column i is row i of R over the original columns, zero past them
+#pragma unroll
+  for (int e = 0; e < RL; ++e) {
+    const int row = row_of(e);
+    if (row < n) {
+      G[row * LD + c0] = x0[e];
+      G[row * LD + c1] = x1[e];
+    }
+  }
+  __syncthreads();
+  // ---- 3. rotations ------------------------------------------------------------
+  // rotation threshold: above the rounding noise of a length-K dot product
+  const T tol = T(8 * max(K, 8)) * Eps<T>::v;
+  const T itol = T(1) / tol;
+  // The rounds run the round-robin schedule cyclically and stop once n2 - 1
+  // consecutive rounds (every pair once, from any starting round) rotated
+  // nothing.  lastrot_sh holds the latest round that rotated: a wave that reads
+  // it late can only see a later round, which no wave left at.
+  const int n2 = n + (n & 1), P = n2 / 2;
+  int rounds = 0;
+  if (n >= 2) {
+    int ca = g, cb = n2 - 1 - g;
+    for (;;) {
+      ++rounds;
+      const int i = min(ca, cb), j = max(ca, cb);
+      if (g < P && j < n) {
+        T x[RL], y[RL];
+        load_col(G + i * LD, x);
+        load_col(G + j * LD, y);
+        const T al = group_sum(dot_tree(x, x), GL), be = group_sum(dot_tree(y, y), GL),
+                ga = group_sum(dot_tree(x, y), GL);
+        const T gt = ga * itol;  // |ga| > tol sqrt(al be), squared with no underflow (al, be > tiny)
+        if (al > tiny && be > tiny && gt * gt > al * be) {
+          T vx[RL], vy[RL];
+          if constexpr (!VG) {
+            load_col(Vs + i * LD, vx);
+            load_col(Vs + j * LD, vy);
+          }
+          T cth, sth;
+          jacobi_rotation(al, be, ga, cth, sth);
+#pragma unroll
+          for (int e = 0; e < RL; ++e) {
+            const T a = x[e], b = y[e];
+            x[e] = cth * a - sth * b;
+            y[e] = sth * a + cth * b;
+          }
+          store_col(G + i * LD, x);
+          store_col(G + j * LD, y);
+          if constexpr (!VG) {
+#pragma unroll
+            for (int e = 0; e < RL; ++e) {
+              const T a = vx[e], b = vy[e];
+              vx[e] = cth * a - sth * b;
+              vy[e] = sth * a + cth * b;
+            }
+            store_col(Vs + i * LD, vx);
+            store_col(Vs + j * LD, vy);
+          }
+          if (sub == 0) lastrot_sh = rounds;
+        }
+      }
+      if (g != 0) ca = (ca == n2 - 1) ? 1 : ca + 1;
+      cb = (cb == n2 - 1) ? 1 : cb + 1;
+      __syncthreads();
+      if (rounds - lastrot_sh >= n2 - 1 || rounds >= 60 * (n2 - 1)) break;
+    }
+  }
+  const int sweeps = (rounds + n2 - 2) / max(1, n2 - 1);
+  if (tid == 0 && it.stats != nullptr) {
+    // this workgroup's copy of the counters (a line of its own: no contention
+    // between the items of a launch)
     int32_t* st = it.stats + (blockIdx.x % kCounterCopies) * kCounterStride;
     atomicAdd(st, 1);
     atomicAdd(st + 1, sweeps);
     atomicMax(st + 2, sweeps);
   }
-  T nx = T(0), ny = T(0);
-#pragma unroll
-  for (int q = 0; q < NR; ++q) {
-    nx += x[q] * x[q];
-    ny += y[q] * y[q];
-  }
-  nx = sqrt(slot_sum<NL>(nx));
-  ny = sqrt(slot_sum<NL>(ny));
-  // the padding column of odd K started at position K2 - 1 and moved one place
-  // per round along the circle of positions 1 .. K2 - 1
-  const int padpos = (K & 1) ? ((K2 - 2 + rounds) % (K2 - 1)) + 1 : -1;
-  if (g == 0 && act) {
-    sig[pt] = (pt == padpos) ? T(-1) : nx;
-    sig[pb] = (pb == padpos) ? T(-1) : ny;
+  // ---- singular values, their order, the rank ----------------------------------
+  load_col(G + c0 * LD, x0);
+  load_col(G + c1 * LD, x1);
+  q0 = group_sum(dot_tree(x0, x0), GL);
+  q1 = group_sum(dot_tree(x1, x1), GL);
+  const T s0 = (c0 < n) ? sqrt(q0) : T(0), s1 = (c1 < n) ? sqrt(q1) : T(0);
+  if (sub == 0) {
+    sig[c0] = s0;
+    sig[c1] = s1;
+    order[c0] = c0;
+    order[c1] = c1;
   }
   __syncthreads();
-  if (lane < K2) {
-    const T sj = sig[lane];
-    int rk = 0;
-    for (int i = 0; i < K2; ++i) {
+  {
+    int r0 = 0, r1 = 0;
+    for (int i = sub; i < K; i += GL) {
       const T si = sig[i];
-      rk += (si > sj || (si == sj && i < lane)) ? 1 : 0;
+      r0 += (si > s0 || (si == s0 && i < c0)) ? 1 : 0;
+      r1 += (si > s1 || (si == s1 && i < c1)) ? 1 : 0;
     }
-    order[rk] = lane;
-    sigs[rk] = sj;
-    rk_of[lane] = rk;
-  }
-  __syncthreads();
-  int r;
-  if (it.fixed_rank >= 0) {
-    r = min(it.fixed_rank, K);
-  } else {
-    // src/operations/misc/misc.cpp:133-146: the smallest r >= 1 with r = md or
-    // sqrt((md - r) sigma_r^2) <= eps ||sigma||, the error summed term by term
-    const int md = (it.kdim > 0) ? min(it.kdim, K) : K;
-    T ss = T(0);
-    for (int i = 0; i < md; ++i) ss += sigs[i] * sigs[i];
-    const T threshold = static_cast<T>(it.eps) * sqrt(ss);
-    bool stop = lane >= 1;
-    if (lane >= 1 && lane < md) {
-      const T sr = sigs[lane];
-      T err = T(0);
-      for (int jj = lane; jj < md; ++jj) err += sr * sr;
-      stop = !(sqrt(err) > threshold);
-    }
-    r = __ffsll((unsigned long long)__ballot(stop)) - 1;
-  }
-  int rout = r;
-  if (r > it.cap) {
-    rout = it.cap_trunc ? it.cap : -r;
-    r = it.cap;
-  }
-  if (lane == 0 && it.rank_out) *it.rank_out = rout;
-  if (nx > T(0)) {
-#pragma unroll
-    for (int q = 0; q < NR; ++q) x[q] /= nx;
-  }
-  if (ny > T(0)) {
-#pragma unroll
-    for (int q = 0; q < NR; ++q) y[q] /= ny;
-  }
-  // Orthonormal completion of kept left vectors whose singular value is
-  // numerically zero (Jacobi leaves those columns unrotated): two passes of
-  // classical Gram-Schmidt of e_u against the earlier kept vectors, accepted
-  // when the remainder keeps norm^2 > thr, with the resumed descending scan of
-  // svd_kernel (a rejected remainder only shrinks as the span grows; a second
-  // scan with thr = 1/(4K) always accepts one).  Rare: it runs on an LDS copy.
-  const T sig_floor = sqrt(tiny);
-  bool need = false;
-  for (int c = 0; c < r; ++c) need = need || !(sigs[c] > sig_floor);
-  if (need) {
-    if (act) {
-#pragma unroll
-      for (int q = 0; q < NR; ++q) {
-        const int ri = g + NL * q;
-        A1[pt][ri] = x[q];
-        A1[pb][ri] = y[q];
+    r0 = group_isum<GL>(r0);
+    r1 = group_isum<GL>(r1);
+    if (sub == 0) {
+      if (c0 < K) {
+        order[r0] = c0;
+        sigs[r0] = s0;
+      }
+      if (c1 < K) {
+        order[r1] = c1;
+        sigs[r1] = s1;
       }
     }
-    __syncthreads();
-    __shared__ int accept_sh;
-    int u = K - 1;
-    T thr = T(0.25);
-    for (int c = 0; c < r; ++c) {
-      const int src = order[c];
-      if (sigs[c] > sig_floor) continue;
-      for (int tries = 0; tries < 2 * K; ++tries, --u) {
-        if (u < 0) {
-          u = K - 1;
-          thr = T(0.25) / T(K);
+  }
+  // unit right vectors in place
+  if (s0 > T(0)) {
+#pragma unroll
+    for (int e = 0; e < RL; ++e) x0[e] /= s0;
+    store_col(G + c0 * LD, x0);
+  }
+  if (s1 > T(0)) {
+#pragma unroll
+    for (int e = 0; e < RL; ++e) x1[e] /= s1;
+    store_col(G + c1 * LD, x1);
+  }
+  __syncthreads();
+  if (wv == 0) {
+    int r;
+    if (it.fixed_rank >= 0) {
+      r = min(it.fixed_rank, K);
+    } else {
+      // src/operations/misc/misc.cpp:133-146: the smallest r >= 1 with r = md or
+      // sqrt((md - r) sigma_r^2) <= eps ||sigma||, the error summed term by term;
+      // a lane per candidate
+      const int md = (it.kdim > 0) ? min(it.kdim, K) : K;
+      T ss = T(0);
+      for (int i = 0; i < md; ++i) ss += sigs[i] * sigs[i];
+      const T threshold = static_cast<T>(it.eps) * sqrt(ss);
+      r = md;
+#pragma unroll
+      for (int k = (KMAX - 1) / 64; k >= 0; --k) {
+        const int cand = lane + 64 * k;
+        bool stop = false;
+        if (cand >= 1 && cand < md) {
+          const T sr = sigs[cand];
+          T err = T(0);
+          for (int jj = cand; jj < md; ++jj) err += sr * sr;
+          stop = !(sqrt(err) > threshold);
         }
-        for (int row = lane; row < K; row += 64) A1[src][row] = (row == u) ? T(1) : T(0);
+        const unsigned long long b = __ballot(stop);
+        if (b) r = 64 * k + __ffsll(b) - 1;
+      }
+      r = max(r, 1);
+    }
+    if (lane == 0) {
+      if (r > it.cap) {
+        if (it.rank_out) *it.rank_out = it.cap_trunc ? it.cap : -r;
+        r = it.cap;
+      } else if (it.rank_out) {
+        *it.rank_out = r;
+      }
+      rank_sh = r;
+    }
+  }
+  __syncthreads();
+  const int r = rank_sh;
+  // Orthonormal completion of kept right vectors whose singular value is
+  // numerically zero (Jacobi leaves those columns unrotated, and the QR drops
+  // them): two passes of classical Gram-Schmidt of e_u against the earlier kept
+  // vectors, accepted when the remainder keeps norm^2 > thr.  Candidates are
+  // scanned from u = K - 1 down and the scan resumes where the previous column's
+  // stopped: a rejected remainder only shrinks as the span grows, and an
+  // accepted e_u lies in it.  The remainders' squared norms sum to K - c, so a
+  // second scan with thr = 1/(4K) always accepts one.
+  const T sig_floor = sqrt(tiny);
+  int u = K - 1;
+  T thr = T(0.25);
+  for (int c = 0; c < r; ++c) {
+    const int src = order[c];
+    if (sigs[c] > sig_floor) continue;
+    for (int tries = 0; tries < 2 * K; ++tries, --u) {
+      if (u < 0) {
+        u = K - 1;
+        thr = T(0.25) / T(K);
+      }
+      for (int row = tid; row < KMAX; row += NT) G[src * LD + row] = (row == u) ? T(1) : T(0);
+      __syncthreads();
+      for (int pass = 0; pass < 2; ++pass) {
+        T xs[RL];
+        load_col(G + src * LD, xs);
+        for (int pp = g; pp < c; pp += NG) {
+          T w[RL];
+          load_col(G + order[pp] * LD, w);
+          const T d = group_sum(dot_tree(w, xs), GL);
+          if (sub == 0) coef[pp] = d;
+        }
         __syncthreads();
-        for (int pass = 0; pass < 2; ++pass) {
-          for (int pp = lane; pp < c; pp += 64) {
-            const int ps = order[pp];
-            T d = T(0);
-            for (int row = 0; row < K; ++row) d += A1[ps][row] * A1[src][row];
-            coef[pp] = d;
-          }
-          __syncthreads();
-          for (int row = lane; row < K; row += 64) {
-            T v = A1[src][row];
-            for (int pp = 0; pp < c; ++pp) v -= coef[pp] * A1[order[pp]][row];
-            A1[src][row] = v;
-          }
-          __syncthreads();
+        for (int row = tid; row < K; row += NT) {
+          T x = G[src * LD + row];
+          for (int pp = 0; pp < c; ++pp) x -= coef[pp] * G[order[pp] * LD + row];
+          G[src * LD + row] = x;
         }
+        __syncthreads();
+      }
+      if (wv == 0) {
+        T nn = T(0);
+        for (int row = lane; row < K; row += 64) nn += G[src * LD + row] * G[src * LD + row];
+        nn = wave_sum(nn);
         if (lane == 0) {
-          T nn = T(0);
-          for (int row = 0; row < K; ++row) nn += A1[src][row] * A1[src][row];
           accept_sh = nn > thr;
           coef[0] = (nn > T(0)) ? T(1) / sqrt(nn) : T(0);
         }
-        __syncthreads();
-        const int ok = accept_sh;
-        const T inv = coef[0];
-        __syncthreads();
-        if (ok) {
-          for (int row = lane; row < K; row += 64) A1[src][row] *= inv;
-          __syncthreads();
-          --u;
-          break;
-        }
       }
-    }
-    if (act) {
-#pragma unroll
-      for (int q = 0; q < NR; ++q) {
-        const int ri = g + NL * q;
-        x[q] = A1[pt][ri];
-        y[q] = A1[pb][ri];
+      __syncthreads();
+      const int ok = accept_sh;
+      const T inv = coef[0];
+      __syncthreads();
+      if (ok) {
+        for (int row = tid; row < K; row += NT) G[src * LD + row] *= inv;
+        __syncthreads();
+        --u;
+        break;
       }
     }
   }
   T* S = static_cast<T*>(it.S);
   T* Um = static_cast<T*>(it.Um);
   T* Vm = static_cast<T*>(it.Vm);
-  if (S != nullptr) {
-#pragma unroll
-    for (int k = 0; k < KMAX * KMAX / 64; ++k) {
-      const int e = lane + 64 * k;
-      const int i = e / KMAX, j = e % KMAX;
-      if (i < r && j < r) S[i * it.lds + j] = (i == j) ? sigs[i] * unscale : T(0);
+  if (S != nullptr)
+    for (int e = tid; e < r * r; e += NT) {
+      const int i = e / r, j = e - (e / r) * r;
+      S[i * it.lds + j] = (i == j) ? sigs[i] * unscale : T(0);
+    }
+  for (int e = tid; e < K * r; e += NT) {
+    const int row = e / r, c = e - (e / r) * r;
+    if (Vm != nullptr) Vm[row * it.ldv + c] = G[order[c] * LD + row];
+    if constexpr (!VG) {
+      if (Um != nullptr) Um[row * it.ldu + c] = Vs[order[c] * LD + row];
     }
   }
-  const int ct = act ? rk_of[pt] : KMAX, cb = act ? rk_of[pb] : KMAX;
+  if constexpr (VG) {
+    // u_c = M v_c / sigma_c: 16 x 16 tiles of M V by FP64 MFMA, a wave per tile
+    const int li = lane & 15, lk = lane >> 4;
+    const int tr = (K + 15) / 16, tc = (r + 15) / 16;
+    if (Um != nullptr)
+      for (int o = wv; o < tr * tc; o += NW) {
+        const int i0 = 16 * (o / tc), j0 = 16 * (o % tc);
+        const T* vc = G + order[min(j0 + li, r - 1)] * LD + lk;
+        const T* mc = vg + min(i0 + li, K - 1);
+        d64::d4 acc = {0.0, 0.0, 0.0, 0.0};
+        // (rows of V past K are zero; the last read row of M is clamped)
+#pragma unroll 8
+        for (int k0 = 0; k0 < K; k0 += 4)
+          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(mc[(int64_t)min(k0 + lk, K - 1) * K], vc[k0], acc, 0, 0, 0);
+        const int c = j0 + li;
+        if (c < r) {
+          const T sc = sigs[c];
 #pragma unroll
-  for (int q = 0; q < NR; ++q) {
-    const int ri = g + NL * q;
-    if (ri < K) {
-      if (ct < r) {
-        if (Um != nullptr) Um[ri * it.ldu + ct] = x[q];
-        if (Vm != nullptr) Vm[ri * it.ldv + ct] = vx[q];
+          for (int v = 0; v < 4; ++v) {
+            const int row = i0 + 4 * v + lk;
+            if (row < K) Um[row * it.ldu + c] = (sc > sig_floor) ? acc[v] / sc : T(0);
+          }
+        }
       }
-      if (cb < r) {
-        if (Um != nullptr) Um[ri * it.ldu + cb] = y[q];
-        if (Vm != nullptr) Vm[ri * it.ldv + cb] = vy[q];
-      }
-    }
   }
 }
 
+// The smallest variant that holds the batch's largest core.  Groups of 16 lanes
+// from 32 columns on (8 lanes a group at K <= 32: even, 35.7 against 35.5 ms per
+// N = 32768 FP64 factorization and solve); one wave of 8-lane groups at K <= 16.
 template <typename T, class Src>
 static void launch_svd_src(Src d_items, int n_items, int max_k, hipStream_t s) {
   if (n_items <= 0) return;
+  auto go = [&](auto kmax, auto gl, auto vg) {
+    constexpr int KM = decltype(kmax)::value, GL = decltype(gl)::value;
+    constexpr bool VG = decltype(vg)::value;
+    hipLaunchKernelGGL((svd_kernel<T, KM, GL, VG, Src>), dim3(n_items), dim3(KM / 2 * GL), 0, s, d_items);
+  };
+  using std::integral_constant;
   if (max_k <= 16) {
-    hipLaunchKernelGGL((svd_reg_kernel<T, 16, Src>), dim3(n_items), dim3(64), 0, s, d_items);
-  } else if (max_k <= 32 && sizeof(T) == 8) {
-    hipLaunchKernelGGL((svd_reg_kernel<T, 32, Src>), dim3(n_items), dim3(64), 0, s, d_items);
+    go(integral_constant<int, 16>{}, integral_constant<int, 8>{}, std::false_type{});
   } else if (max_k <= 32) {
-    hipLaunchKernelGGL((svd_kernel<T, 32, 64, false, Src>), dim3(n_items), dim3(64), 0, s, d_items);
+    go(integral_constant<int, 32>{}, integral_constant<int, 16>{}, std::false_type{});
   } else if (max_k <= 64) {
-    hipLaunchKernelGGL((svd_kernel<T, 64, 256, false, Src>), dim3(n_items), dim3(256), 0, s, d_items);
+    go(integral_constant<int, 64>{}, integral_constant<int, 16>{}, std::false_type{});
   } else if (max_k <= 128) {
-    if constexpr (sizeof(T) == 4) {
-      hipLaunchKernelGGL((svd_kernel<T, 128, 1024, false, Src>), dim3(n_items), dim3(1024), 0, s, d_items);
-    } else {
-      // every item must carry a K x K scratch (SvdItem::vwork) for its right vectors
-      hipLaunchKernelGGL((svd_kernel<T, 128, 1024, true, Src>), dim3(n_items), dim3(1024), 0, s, d_items);
-    }
+    // FP64: every item must carry a K x K scratch (SvdItem::vwork)
+    go(integral_constant<int, 128>{}, integral_constant<int, 16>{}, std::bool_constant<(sizeof(T) == 8)>{});
   } else {
     throw std::runtime_error("svd: K above 128");
   }

@@ -1,0 +1,88 @@
+"""Cores of the batched low-rank addition at the edges of the Jacobi SVD kernel's
+variants (16, 32, 64 and 128 columns; FP64 above 64 keeps one array in LDS), with the
+spectra that take its different ways: full numerical rank, a tail the pivoted QR drops,
+numerically rank-deficient cores kept at a larger fixed rank, and zero."""
+import numpy as np
+import pytest
+
+from oracle import frank_oracle as fo
+
+pytestmark = pytest.mark.gpu
+
+
+def _pair(rng, m, n, k1, k2, decay, common):
+    """Two factored matrices (orthonormal bases, singular values 10^(-decay i)); with
+    common bases the sum has numerical rank max(k1, k2)."""
+    q = lambda rows, k: np.linalg.qr(rng.standard_normal((rows, k)))[0]
+    s = lambda k: np.diag(10.0 ** (-decay * np.arange(k)))
+    if common:
+        k = max(k1, k2)
+        U, V = q(m, k), q(n, k)
+        U2, V2 = U, V
+    else:
+        U, V, U2, V2 = q(m, k1), q(n, k1), q(m, k2), q(n, k2)
+    return (U[:, :k1], s(k1), V[:, :k1].T), (U2[:, :k2], s(k2), V2[:, :k2].T)
+
+
+def _add(torch, fa, pairs, cap, eps, dtype):
+    As, Bs = [], []
+    for (U, S, V), B in pairs:
+        m, k = U.shape
+        slot = lambda r, c, x: torch.nn.functional.pad(torch.from_numpy(np.ascontiguousarray(x)),
+                                                       (0, c - x.shape[1], 0, r - x.shape[0])).to("cuda", dtype)
+        As.append((slot(m, cap, U), slot(cap, cap, S), slot(cap, V.shape[1], V), k))
+        Bs.append(tuple(torch.from_numpy(np.ascontiguousarray(x)).to("cuda", dtype) for x in B))
+    ranks = fa.lr_add_batched(As, Bs, eps=eps, lra="rounded_addition", cap=cap)
+    return [tuple(x.double().cpu().numpy() for x in (a[0][:, :r], a[1][:r, :r], a[2][:r])) for a, r in zip(As, ranks)]
+
+
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("k1,k2", [(1, 1), (2, 1), (8, 8), (9, 8), (16, 15), (16, 16), (17, 16), (31, 32), (32, 32),
+                                   (33, 32), (64, 63), (64, 64)])
+@pytest.mark.parametrize("decay", [0.05, 0.2])
+def test_core_sizes(torch_gpu, fa, dtype, k1, k2, decay):
+    print(f"cores {dtype} {k1}+{k2} decay {decay}", flush=True)
+    torch = torch_gpu
+    rng = np.random.default_rng(100 * k1 + k2)
+    u = np.finfo(dtype).eps
+    eps = 1e-9 if dtype == "float64" else 1e-5
+    pairs = [_pair(rng, 200, 150, k1, k2, decay, c) for c in (False, True)]
+    for (A, B), (U, S, V) in zip(pairs, _add(torch, fa, pairs, 128, eps, getattr(torch, dtype))):
+        D = (A[0] @ A[1]) @ A[2] + (B[0] @ B[1]) @ B[2]
+        sv = np.linalg.svd(D, compute_uv=False)
+        K = k1 + k2
+        r = U.shape[1]
+        # the truncation rule keeps sqrt(K - r) sigma_r <= eps ||sigma||; the tail is at most that, and
+        # rounding (QR of both panels, the core's products and rotations) some K u on top
+        err = np.linalg.norm(D - (U @ S) @ V)
+        assert err <= (1.01 * eps + 8 * K * u) * np.linalg.norm(sv)
+        assert np.linalg.norm(sv[r:]) <= (eps + 8 * K * u) * np.linalg.norm(sv)
+        assert np.abs(np.diag(S) - sv[:r]).max() <= 8 * K * u * sv[0]
+        # right vectors: pairwise orthogonal to the rotation threshold 8 max(K, 8) u
+        assert np.abs(V @ V.T - np.eye(r)).max() <= 16 * max(K, 8) * u
+        if not (dtype == "float64" and K > 64):  # that variant forms u = M v / sigma: ||M|| / sigma_r times u
+            assert np.abs(U.T @ U - np.eye(r)).max() <= 16 * max(K, 8) * u
+        # the oracle's rank, where the decision is not within rounding of the threshold
+        want = fo.find_svd_truncation_rank(sv[:min(K, len(sv))], eps)
+        if dtype == "float64":
+            assert r == want
+
+
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("k1,k2", [(2, 2), (8, 8), (12, 20), (24, 24), (30, 34)])
+def test_fixed_rank_above_the_numerical_rank(torch_gpu, fa, dtype, k1, k2):
+    """eps = 0 keeps rank k1 although the sum's numerical rank is far smaller: the missing
+    vectors of both bases are completed to orthonormal sets.  Also the zero core."""
+    print(f"fixed rank {dtype} {k1}+{k2}", flush=True)
+    torch = torch_gpu
+    rng = np.random.default_rng(k1)
+    u = np.finfo(dtype).eps
+    A, B = _pair(rng, 160, 130, k1, k2, 4.0, True)  # numerical rank at most 5
+    Z = (A[0], 0 * A[1], A[2]), (B[0], 0 * B[1], B[2])
+    for (P, Q), (U, S, V) in zip([(A, B), Z], _add(torch, fa, [(A, B), Z], 64, 0.0, getattr(torch, dtype))):
+        D = (P[0] @ P[1]) @ P[2] + (Q[0] @ Q[1]) @ Q[2]
+        K = k1 + k2
+        assert U.shape[1] == k1
+        assert np.linalg.norm(D - (U @ S) @ V) <= 8 * K * u * np.linalg.norm(D)
+        assert np.abs(V @ V.T - np.eye(k1)).max() <= 16 * max(K, 8) * u
+        assert np.abs(U.T @ U - np.eye(k1)).max() <= 16 * max(K, 8) * u
