@@ -758,8 +758,10 @@ __global__ __launch_bounds__(256) void tile_lu_kernel(TileLuItem it) {
     blk_load32(M, it.a32_in + off_a, ld, mi, nj);
   else
     blk_load(M, Ablk, ld, mi, nj);
-  if (bi == bj)
+  if (bi == bj && mi < 64) {
+    __syncthreads();  // the load above zeroes these elements from other threads
     for (int r = mi + tid; r < 64; r += 256) M[r * LD + r] = 1.0;  // identity padding of the last diagonal block
+  }
   if (it.pre_core != nullptr) {
     // 0. the low-rank update of the tile, on this block: M += U_blk (core V_blk)
     __syncthreads();
