@@ -807,7 +807,7 @@ void lr_add_batched_impl(frk_ctx ctx, int lra, int batch, const int32_t* m, cons
     mmax = std::max(mmax, m[b]);
     nmax = std::max(nmax, n[b]);
   }
-  need += (size_t)batch * sizeof(T) * ((size_t)(mmax + nmax) * kmax + 6 * (size_t)kmax * kmax + 2 * kmax + 512);
+  need += lr_add_bound<T>(batch, mmax, nmax, kmax);
   c.reserve(need);
   for (int b = 0; b < batch; ++b) {
     LrAddDesc<T> x{};

@@ -216,7 +216,8 @@ struct LrAddDesc {
 };
 
 // Per-batch workspace of a batched low-rank addition: addition t owns
-// Yu/Yv + t*mmax*K / t*nmax*K (reflectors), tu/tv + t*K, Ru/Rv/Um/Vm + t*K*K
+// Yu/Yv + t*mmax*K / t*nmax*K (reflectors), tu/tv + t*K (these with Kp = 0; the
+// blocked kernels' layout below), Ru/Rv/Um/Vm + t*K*K
 // (and Vw, Mw + t*K*K when set).  lra: 1 rounded, 2 fast (when eps == 0).
 // An addition whose K = kc + kx2 exceeds a tile dimension has a core of
 // Ke = max(min(m, K), min(n, K)) < K: its M = Ru Rv^T (Ke x Ke) is formed into
@@ -226,7 +227,12 @@ struct LrBatch {
   T *Yu, *Yv, *tu, *tv, *Ru, *Rv, *Um, *Vm, *Vw, *Mw;
   int32_t* stats;
   int32_t mmax, nmax, K, lra;
-  int32_t Kmax_svd, pad;
+  int32_t Kmax_svd;
+  // the blocked QR / basis update (lr_qr.hip): rows (a multiple of 16) and columns
+  // (K rounded up to 16) of each addition's reflector buffer; its tu / tv slots hold
+  // the 16 x 16 triangular factors of the panels.  Kp = 0: the unblocked kernels'
+  // layout (m x K reflectors, K scalars).
+  int32_t ldu, ldv, Kp;
 };
 
 // ---------------------------------------------------------------------------

@@ -642,22 +642,6 @@ void trsm_generic(const T* A, int64_t a_rs, int64_t a_cs, bool lower, bool unit,
 // Rounded low-rank addition (batched)
 // ============================================================================
 template <typename T>
-size_t lr_add_workspace(const std::vector<LrAddDesc<T>>& d) {
-  int kmax = 0, mmax = 0, nmax = 0;
-  for (const auto& x : d) {
-    kmax = std::max(kmax, x.kc + x.kx2);
-    mmax = std::max(mmax, x.m);
-    nmax = std::max(nmax, x.n);
-  }
-  const size_t K = kmax;
-  const size_t vw = (sizeof(T) == 8 && K > 64) ? K * K : 0;  // Jacobi right-vector scratch
-  bool small_core = false;                                   // a core formed before its SVD
-  for (const auto& x : d) small_core = small_core || x.kc + x.kx2 > std::min(x.m, x.n);
-  const size_t mw = small_core ? K * K : 0;
-  return d.size() * sizeof(T) * ((size_t)(mmax + nmax) * K + 2 * K + 4 * K * K + vw + mw) + 10 * 256 + 4096;
-}
-
-template <typename T>
 void plan_lr_add(Plan& pl, const std::vector<LrAddDesc<T>>& d_in, int lra) {
   if (d_in.empty()) return;
   Context& ctx = pl.ctx();
@@ -730,10 +714,30 @@ void plan_lr_add(Plan& pl, const std::vector<LrAddDesc<T>>& d_in, int lra) {
     cls_kmax[c] = std::max(cls_kmax[c], Ke);
   }
   LrBatch<T> b{};
-  b.Yu = ctx.take<T>((size_t)nd * mmax * K);
-  b.Yv = ctx.take<T>((size_t)nd * nmax * K);
-  b.tu = ctx.take<T>((size_t)nd * K);
-  b.tv = ctx.take<T>((size_t)nd * K);
+  // the blocked QR and basis update address an operand with 31-bit byte offsets
+  bool near = true;
+  auto reach = [&](int64_t r, int64_t rs, int64_t c, int64_t cs) {
+    if (r <= 0 || c <= 0) return;
+    constexpr int64_t lim = (int64_t)0x7fffff00 / (int64_t)sizeof(T);
+    near = near && rs >= 0 && cs >= 0 && rs < lim && cs < lim && (r - 1) * rs + (c - 1) * cs < lim;
+  };
+  for (const auto& x : d) {
+    reach(x.m, x.cu_rs, x.kc, x.cu_cs);
+    reach(x.kc, x.cv_rs, x.n, x.cv_cs);
+    reach(x.kc, x.lds, x.kc, 1);
+    reach(x.m, x.xu_rs, x.kx1, x.xu_cs);
+    reach(x.kx1, x.xs_ld, x.kx2, 1);
+    reach(x.kx2, x.xv_rs, x.n, x.xv_cs);
+  }
+  if (near && lr_blocked_ok<T>(nd, std::max(mmax, nmax), std::max(qk, capmax))) {
+    b.Kp = (K + 15) / 16 * 16;
+    b.ldu = (mmax + 15) / 16 * 16;
+    b.ldv = (nmax + 15) / 16 * 16;
+  }
+  b.Yu = ctx.take<T>((size_t)nd * (b.Kp ? b.ldu * b.Kp : mmax * K));
+  b.Yv = ctx.take<T>((size_t)nd * (b.Kp ? b.ldv * b.Kp : nmax * K));
+  b.tu = ctx.take<T>((size_t)nd * (b.Kp ? 16 * b.Kp : K));
+  b.tv = ctx.take<T>((size_t)nd * (b.Kp ? 16 * b.Kp : K));
   b.Ru = ctx.take<T>((size_t)nd * K * K);
   b.Rv = ctx.take<T>((size_t)nd * K * K);
   b.Um = ctx.take<T>((size_t)nd * K * K);
@@ -1814,7 +1818,7 @@ void blr_getrf(BlrMatrix<T>& A, Context& ctx, int max_steps) {
           need += sizeof(T) * ((size_t)bm * kmax + (size_t)kmax * kmax + 512);
         if (kc == kLowRank) {
           const size_t K = (size_t)kmax + ((kl == kDense && kb == kDense) ? (size_t)A.kcap : (size_t)kmax);
-          need += sizeof(T) * (2 * bm * K + 2 * K + 6 * K * K) + 10 * 256;
+          need += sizeof(T) * (lr_qr_elems(bm, bm, K) + 6 * K * K) + 10 * 256;
         }
       }
     return need;
@@ -2907,7 +2911,6 @@ RefineResult blr_refine(BlrMatrix<T>& F, const KernelSpec& ks, double anorm, con
 #define FRK_ENGINE_INST(T)                                                                                  \
   template class BlrMatrix<T>;                                                                              \
   template void plan_lr_add<T>(Plan&, const std::vector<LrAddDesc<T>>&, int);                               \
-  template size_t lr_add_workspace<T>(const std::vector<LrAddDesc<T>>&);                                    \
   template void lr_add_batched<T>(const std::vector<LrAddDesc<T>>&, int, Context&);                         \
   template void lr_add_naive<T>(const std::vector<LrAddDesc<T>>&, Context&);                                \
   template void compress_batched<T>(const std::vector<CompressDesc<T>>&, Context&);                         \

@@ -281,11 +281,9 @@ class BlrMatrix {
 // ----------------------------------------------------------------------------
 
 // C += X for every descriptor (reference: rounded_addition / fast_rounded_addition).
-// Workspace comes from the plan's context (reserve lr_add_workspace() first).
+// Workspace comes from the plan's context (reserve lr_add_bound() first).
 template <typename T>
 void plan_lr_add(Plan& pl, const std::vector<LrAddDesc<T>>& d, int lra);
-template <typename T>
-size_t lr_add_workspace(const std::vector<LrAddDesc<T>>& d);
 template <typename T>
 void lr_add_batched(const std::vector<LrAddDesc<T>>& d, int lra, Context& ctx);
 // naive_addition: concatenation, dense recompression past min(m, n).  Synchronous.
@@ -447,10 +445,16 @@ void typed_gemm(TypedBatch<T>& b, Context& ctx, const Op<T>& A, const Op<T>& B, 
 template <typename T>
 void run_typed_batch(TypedBatch<T>& b, Context& ctx, int lra);
 
+// Elements of one addition's reflectors and their triangular factors, rows and
+// columns rounded up to tiles of 16 (the unblocked layout needs less).
+inline size_t lr_qr_elems(size_t m, size_t n, size_t K) {
+  const size_t Kp = (K + 15) / 16 * 16;
+  return ((m + 15) / 16 * 16 + (n + 15) / 16 * 16 + 32) * Kp;
+}
 // Workspace bound of plan_lr_add for nd additions of at most m x n with K columns.
 template <typename T>
 size_t lr_add_bound(int nd, int m, int n, int K) {
-  return (size_t)nd * sizeof(T) * ((size_t)(m + n) * K + 2 * (size_t)K + 6 * (size_t)K * K) + 10 * 256 + 4096;
+  return (size_t)nd * sizeof(T) * (lr_qr_elems(m, n, K) + 6 * (size_t)K * K) + 10 * 256 + 4096;
 }
 
 // ----------------------------------------------------------------------------
