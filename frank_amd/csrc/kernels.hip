@@ -2191,61 +2191,6 @@ void launch_lr_add_qr(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, int ma
   else
     launch_qr_src<T>(LrQrItems<T>{d, b}, 2 * nd, max_k, s, std::max(b.mmax, b.nmax));
 }
-// M = Ru Rv^T (Ke x Ke, row stride K) of the additions whose core is smaller
-// than K = kc + kx2 (a workgroup each; the others return at once): Ru and Rv
-// staged through LDS in chunks of 32 of the K columns.
-template <typename T>
-__global__ __launch_bounds__(256) void lr_core_prod_kernel(const LrAddDesc<T>* __restrict__ d, LrBatch<T> b) {
-  const int t = blockIdx.x;
-  const LrAddDesc<T> x = d[t];
-  const int K = b.K, Kt = x.kc + x.kx2, Ke = lr_core_dim(x, b);
-  if (Ke >= Kt) return;
-  constexpr int QC = 32, NO = 128 * 128 / 256;
-  __shared__ T Us[128][QC + 1];
-  __shared__ T Vs[128][QC + 1];
-  const T* Ru = b.Ru + (size_t)t * K * K;
-  const T* Rv = b.Rv + (size_t)t * K * K;
-  T* M = b.Mw + (size_t)t * K * K;
-  const int tid = threadIdx.x;
-  T acc[NO];
-#pragma unroll
-  for (int k = 0; k < NO; ++k) acc[k] = T(0);
-  for (int q0 = 0; q0 < Kt; q0 += QC) {
-    __syncthreads();
-    for (int e = tid; e < Ke * QC; e += 256) {
-      const int i = e / QC, q = e % QC;
-      const bool in = q0 + q < Kt;
-      Us[i][q] = in ? Ru[(int64_t)i * K + q0 + q] : T(0);
-      Vs[i][q] = in ? Rv[(int64_t)i * K + q0 + q] : T(0);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < NO; ++k) {
-      const int e = tid + 256 * k;
-      if (e < Ke * Ke) {
-        const int i = e / Ke, j = e - (e / Ke) * Ke;
-        T a = acc[k];
-#pragma unroll 8
-        for (int q = 0; q < QC; ++q) a += Us[i][q] * Vs[j][q];
-        acc[k] = a;
-      }
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < NO; ++k) {
-    const int e = tid + 256 * k;
-    if (e < Ke * Ke) M[(int64_t)(e / Ke) * K + e % Ke] = acc[k];
-  }
-}
-
-template <typename T>
-void launch_lr_add_core(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, hipStream_t s) {
-  if (nd <= 0 || b.Mw == nullptr) return;
-  if (b.K > 128) throw std::runtime_error("lr core product: K above 128");
-  hipLaunchKernelGGL(lr_core_prod_kernel<T>, dim3(nd), dim3(256), 0, s, d, b);
-  FRK_HIP_CHECK(hipGetLastError());
-}
-
 template <typename T>
 void launch_lr_add_svd(const LrAddDesc<T>* d, int t0, int n, int max_k, const LrBatch<T>& b, hipStream_t s) {
   launch_svd_src<T>(LrSvdItems<T>{d, b, t0}, n, max_k, s);
@@ -3727,7 +3672,6 @@ template void launch_axpy_convert<float>(double*, const float*, int64_t, hipStre
   template void launch_svd<T>(const SvdItem*, int, int, hipStream_t);                            \
   template void launch_lr_add_qr<T>(const LrAddDesc<T>*, int, const LrBatch<T>&, int, hipStream_t);  \
   template void launch_lr_add_svd<T>(const LrAddDesc<T>*, int, int, int, const LrBatch<T>&, hipStream_t); \
-  template void launch_lr_add_core<T>(const LrAddDesc<T>*, int, const LrBatch<T>&, hipStream_t);     \
   template void launch_lr_add_apply<T>(const LrAddDesc<T>*, int, const LrBatch<T>&, int, hipStream_t); \
   template void launch_geqp3<T>(const Geqp3Item*, int, hipStream_t);                             \
   template void launch_permute_r<T>(const PermuteItem*, int, int, int, hipStream_t);             \

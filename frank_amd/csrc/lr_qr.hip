@@ -657,6 +657,51 @@ __global__ __launch_bounds__(64 * NW * RW) void lr_apply_kernel(Src items) {
   }
 }
 
+// M = Ru Rv^T (Ke x Ke, row stride K) of the additions whose core is smaller than
+// K = kc + kx2 (a workgroup each; the others return at once).  Wave w forms the tile
+// rows w and w + 4: a lane reads four consecutive columns of its row of Ru and of a
+// row of Rv per tile, and the MFMA products take them as the contraction index (any
+// order will do, if both operands have the same).  Both are upper trapezoidal, so a
+// tile row starts at its diagonal tile.  Bound by the FP64 MFMA rate of one CU and the
+// latency of the reads.  FP64, 165 cores of 64 from 128 columns: 26 us, 135 us with
+// the factors staged through LDS and one FMA a pair of LDS reads.
+template <typename T, int NJ>
+__global__ __launch_bounds__(256) void lr_core_prod_kernel(const LrAddDesc<T>* __restrict__ d, LrBatch<T> b) {
+  using M = Mma<T>;
+  using v4 = typename M::v4;
+  const int t = blockIdx.x;
+  const LrAddDesc<T> x = d[t];
+  const int K = b.K, Kt = x.kc + x.kx2, Ke = lr_core_dim(x, b);
+  if (Ke >= Kt) return;
+  const Buf<T> Ru(b.Ru + (size_t)t * K * K), Rv(b.Rv + (size_t)t * K * K), Mo(b.Mw + (size_t)t * K * K);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, lr = lane >> 4;
+  for (int i = w; 16 * i < Ke; i += 4) {
+    v4 acc[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[j] = v4{0, 0, 0, 0};
+#pragma unroll 1
+    for (int q = 16 * i + 4 * lr; __any(q < Kt); q += 16) {
+      const int ra = 16 * i + M::irow(li);
+      v4 a = Ru.load4(at<T>(ra < Ke, ra, K, q, 1)), v[NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) v[j] = Rv.load4(at<T>(16 * j + li < Ke, 16 * j + li, K, q, 1));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const T ae = (q + e < Kt) ? a[e] : T(0);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[j] = M::mma(ae, (q + e < Kt) ? v[j][e] : T(0), acc[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = 16 * i + 4 * lr + e, col = 16 * j + li;
+        Mo.store(at<T>(row < Ke && col < Ke, row, K, col, 1), acc[j][e]);
+      }
+  }
+}
+
 template <typename T, int NT, int RW, int NP>
 void qr_go(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, hipStream_t s) {
   hipLaunchKernelGGL((lr_qr_kernel<T, NT, RW, NP, LrQrItems<T>>), dim3(2 * nd), dim3(64 * NP * RW), 0, s,
@@ -736,10 +781,22 @@ void launch_lr_apply_blocked(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b,
   FRK_HIP_CHECK(hipGetLastError());
 }
 
+template <typename T>
+void launch_lr_add_core(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, hipStream_t s) {
+  if (nd <= 0 || b.Mw == nullptr) return;
+  if (b.K > 128) throw std::runtime_error("lr core product: K above 128");
+  if (b.Kmax_svd <= 64)
+    hipLaunchKernelGGL((lr_core_prod_kernel<T, 4>), dim3(nd), dim3(256), 0, s, d, b);
+  else
+    hipLaunchKernelGGL((lr_core_prod_kernel<T, 8>), dim3(nd), dim3(256), 0, s, d, b);
+  FRK_HIP_CHECK(hipGetLastError());
+}
+
 #define FRK_LRQR_INST(T)                                                                                   \
   template bool lr_blocked_ok<T>(int, int, int);                                                                \
   template void launch_lr_qr_blocked<T>(const LrAddDesc<T>*, int, const LrBatch<T>&, int, hipStream_t);    \
-  template void launch_lr_apply_blocked<T>(const LrAddDesc<T>*, int, const LrBatch<T>&, int, hipStream_t);
+  template void launch_lr_apply_blocked<T>(const LrAddDesc<T>*, int, const LrBatch<T>&, int, hipStream_t); \
+  template void launch_lr_add_core<T>(const LrAddDesc<T>*, int, const LrBatch<T>&, hipStream_t);
 FRK_LRQR_INST(double)
 FRK_LRQR_INST(float)
 
