@@ -2204,19 +2204,33 @@ void launch_lr_add_apply(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, int
 }
 
 // ===========================================================================
-// Truncated column-pivoted Householder QR (geqp3 with LAWN-176 downdating),
-// one 512-thread workgroup per row-major tile; thread-per-column sweeps.
+// Truncated column-pivoted Householder QR (geqp3 with LAWN-176 downdating), one
+// 512-thread workgroup per row-major tile, thread c for column c (and for row c of the
+// pivot column).  The reflectors' updates are deferred, as in LAPACK's laqps: with
+// F = A^T V T of the last up to B reflectors, a step reads the tile once (the products
+// of the new reflector with every column, which for the columns of the earlier
+// reflectors are the entries of V^T v), and only the pivot column and row r are brought
+// up to date; the tile is rewritten once in B steps.  A column's entries of F, its norms
+// and its index stay in its thread's registers.
+// Bound by memory: 992 tiles of 512 x 512 (2 MiB each, 256 at a time) do not fit the
+// caches; read about once a step they take 5.3 ms at ranks near 11 (12.8 ms with two
+// reads and a write a step; 9.4 ms with the norms formed anew from V in global memory,
+// which most columns need twice).
 // ===========================================================================
 template <typename T>
-__device__ T block_sum512(T v, T* red) {
-  const int tid = threadIdx.x;
-  red[tid] = v;
+__device__ __forceinline__ T wave_sum64(T v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  return v;
+}
+template <typename T>
+__device__ T block_sum512(T v, T* red8) {
+  v = wave_sum64(v);
+  if ((threadIdx.x & 63) == 0) red8[threadIdx.x >> 6] = v;
   __syncthreads();
-  for (int s = 256; s > 0; s >>= 1) {
-    if (tid < s) red[tid] = red[tid] + red[tid + s];
-    __syncthreads();
-  }
-  const T out = red[0];
+  T out = T(0);
+#pragma unroll
+  for (int w = 0; w < 8; ++w) out += red8[w];
   __syncthreads();
   return out;
 }
@@ -2227,54 +2241,98 @@ __global__ __launch_bounds__(512) void geqp3_kernel(const Geqp3Item* __restrict_
   T* A = static_cast<T*>(it.A);
   const int m = it.m, n = it.n;
   const int64_t lda = it.lda;
-  const int tid = threadIdx.x;
-  __shared__ T cn[512], pcn[512], vv[512], red[512];
-  __shared__ int piv[512], redi[512];
+  const int tid = threadIdx.x, c = tid;
+  constexpr int B = 16, VR = 512 / B;
+  __shared__ T vv[512], Vs[VR][B], red8[8];
+  __shared__ T fp[B], fr[B], wk[B], vr[B], swp[2], alpha_sh;
+  __shared__ int redi[8], swi;
   const T tol = Eps<T>::half;
   const T tol3z = sqrt(tol);
   const int min_dim = min(m, n);
-  T part = T(0);
-  for (int c = tid; c < n; c += 512) {
-    T s = T(0);
-    for (int i = 0; i < m; ++i) {
-      const T x = A[i * lda + c];
-      s += x * x;
+  const bool col = c < n;
+  T cn = T(0), pcn;
+  int pc = c;
+  // rows >= r of the columns >= r: A(i, c) - sum_k V(i, k) F(c, k), V(i, k) = A(i, r0 + k), k < r - r0
+  T f[B];
+#pragma unroll
+  for (int k = 0; k < B; ++k) f[k] = T(0);
+  // products of rows r0.. of column c with x (x in LDS; null: with itself)
+  auto column_dot = [&](int r0, const T* x) {
+    T s[4] = {T(0), T(0), T(0), T(0)};
+    const T* p = A + c;
+    int i = r0;
+    for (; i + 16 <= m; i += 16) {
+      T a[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) a[u] = p[(i + u) * lda];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) s[u & 3] += (x ? x[i + u] : a[u]) * a[u];
     }
-    part += s;
-    cn[c] = sqrt(s);
-    pcn[c] = cn[c];
-    piv[c] = c;
-  }
-  const T total = block_sum512(part, red);
-  const T threshold = static_cast<T>(it.eps) * sqrt(total);
-  T* tau_out = static_cast<T*>(it.tau);
-  // initial max
-  auto block_argmax = [&](int from, T& best, int& besti) {
-    T bv = -T(1);
-    int bi = 0x7fffffff;
-    for (int c = from + tid; c < n; c += 512) {
-      const T x = cn[c];
-      if (x > bv || (x == bv && c < bi)) {
-        bv = x;
-        bi = c;
-      }
+    for (; i < m; ++i) {
+      const T a = p[i * lda];
+      s[0] += (x ? x[i] : a) * a;
     }
-    red[tid] = bv;
-    redi[tid] = bi;
-    __syncthreads();
-    for (int s = 256; s > 0; s >>= 1) {
-      if (tid < s) {
-        const T o = red[tid + s];
-        const int oi = redi[tid + s];
-        if (o > red[tid] || (o == red[tid] && oi < redi[tid])) {
-          red[tid] = o;
-          redi[tid] = oi;
+    return (s[0] + s[1]) + (s[2] + s[3]);
+  };
+  // column c's rows i0.. with the deferred updates, VR rows of V staged at a time: take(i, value)
+  auto updated_column = [&](int i0, int r0, int kn, bool mine, auto&& take) {
+    for (; i0 < m; i0 += VR) {
+      const int i = i0 + tid / B, k = tid % B;
+      Vs[tid / B][k] = (i < m && k < kn) ? A[i * lda + r0 + k] : T(0);
+      __syncthreads();
+      if (mine) {
+        const int nr = min(VR, m - i0);
+        const T* q = A + i0 * lda + c;
+        for (int j0 = 0; j0 < nr; j0 += 8) {
+          T x[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) x[u] = q[min(j0 + u, nr - 1) * lda];
+#pragma unroll
+          for (int u = 0; u < 8; ++u)
+            if (j0 + u < nr) {
+#pragma unroll
+              for (int k = 0; k < B; ++k) x[u] -= Vs[j0 + u][k] * f[k];
+              take(i0 + j0 + u, x[u]);
+            }
         }
       }
       __syncthreads();
     }
-    best = red[0];
+  };
+  T part = T(0);
+  if (col) {
+    part = column_dot(0, nullptr);
+    cn = sqrt(part);
+  }
+  pcn = cn;
+  const T total = block_sum512(part, red8);
+  const T threshold = static_cast<T>(it.eps) * sqrt(total);
+  T* tau_out = static_cast<T*>(it.tau);
+  // the first maximum of the norms of the columns from `from` on (a NaN is never one)
+  auto block_argmax = [&](int from, T& best, int& besti) {
+    T bv = (col && c >= from && cn > -T(1)) ? cn : -T(1);
+    int bi = bv > -T(1) ? c : 0x7fffffff;
+    auto better = [](T o, int oi, T& v, int& vi) {
+      if (o > v || (o == v && oi < vi)) {
+        v = o;
+        vi = oi;
+      }
+    };
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const T ov = __shfl_xor(bv, o);
+      const int oi = __shfl_xor(bi, o);
+      better(ov, oi, bv, bi);
+    }
+    if ((tid & 63) == 0) {
+      red8[tid >> 6] = bv;
+      redi[tid >> 6] = bi;
+    }
+    __syncthreads();
+    best = red8[0];
     besti = redi[0];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) better(red8[w], redi[w], best, besti);
     __syncthreads();
   };
   T maxv;
@@ -2282,7 +2340,7 @@ __global__ __launch_bounds__(512) void geqp3_kernel(const Geqp3Item* __restrict_
   block_argmax(0, maxv, kmax);
   if (maxv <= tol) {
     // zero matrix: Q = e1, R = 0 (rank 1)
-    for (int c = tid; c < n; c += 512) {
+    if (col) {
       A[c] = T(0);
       it.piv[c] = c;
     }
@@ -2295,37 +2353,52 @@ __global__ __launch_bounds__(512) void geqp3_kernel(const Geqp3Item* __restrict_
   // eps < 0: exactly min(cap, min_dim) pivot steps (dgeqp3 prefix, used by the ID)
   const bool fixed = it.eps < 0.0;
   const int steps = (fixed || it.cap_trunc) ? min(it.cap, min_dim) : min_dim;
-  int r = 0;
+  int r = 0, r0 = 0;
   while (r < steps && (fixed || maxv > threshold)) {
-    // pivot: first maximum of cn[r:] (computed at the end of the previous step)
-    const int k = kmax;
-    if (k != r) {
-      for (int i = tid; i < m; i += 512) {
-        const T x = A[i * lda + r];
-        A[i * lda + r] = A[i * lda + k];
-        A[i * lda + k] = x;
-      }
+    const int kb = r - r0;
+    const int p = kmax < n ? kmax : r;  // (no maximum: norms of NaN only)
+    // columns r and p change places: the pivot's F to all, column r's to thread p
+    if (c == p) {
+#pragma unroll
+      for (int k = 0; k < B; ++k) fp[k] = f[k];
+      it.piv[r] = pc;
+    }
+    if (c == r) {
+#pragma unroll
+      for (int k = 0; k < B; ++k) fr[k] = f[k];
+      swp[0] = cn;
+      swp[1] = pcn;
+      swi = pc;
     }
     __syncthreads();
-    if (tid == 0 && k != r) {
-      T x = cn[r];
-      cn[r] = cn[k];
-      cn[k] = x;
-      x = pcn[r];
-      pcn[r] = pcn[k];
-      pcn[k] = x;
-      const int pi = piv[r];
-      piv[r] = piv[k];
-      piv[k] = pi;
+    if (c == p && p != r) {
+#pragma unroll
+      for (int k = 0; k < B; ++k) f[k] = fr[k];
+      cn = swp[0];
+      pcn = swp[1];
+      pc = swi;
     }
-    // reflector from column r
-    T x2p = T(0);
-    for (int i = r + 1 + tid; i < m; i += 512) {
-      const T x = A[i * lda + r];
-      x2p += x * x;
+    // the pivot column up to date (thread i: row i)
+    T a = T(0);
+    if (tid < m) {
+      T* Ai = A + tid * lda;
+      a = Ai[p];
+      if (p != r) Ai[p] = Ai[r];
+      if (tid >= r) {
+#pragma unroll
+        for (int k = 0; k < B; ++k)
+          if (k < kb) {
+            const T v = Ai[r0 + k];
+            a -= v * fp[k];
+            if (tid == r) vr[k] = v;
+          }
+      } else if (p != r) {
+        Ai[r] = a;
+      }
+      if (tid == r) alpha_sh = a;
     }
-    const T x2 = (r < m - 1) ? block_sum512(x2p, red) : T(0);
-    const T alpha = A[r * lda + r];
+    const T x2 = block_sum512((tid > r && tid < m) ? a * a : T(0), red8);
+    const T alpha = alpha_sh;
     T beta, tau, scal;
     if (x2 == T(0)) {
       tau = T(0);
@@ -2337,57 +2410,72 @@ __global__ __launch_bounds__(512) void geqp3_kernel(const Geqp3Item* __restrict_
       tau = (beta - alpha) / beta;
       scal = T(1) / (alpha - beta);
     }
-    for (int i = r + 1 + tid; i < m; i += 512) {
-      const T x = A[i * lda + r] * scal;
-      A[i * lda + r] = x;
-      vv[i] = x;
+    if (tid < m && tid >= r) {
+      const T v = (tid == r) ? T(1) : a * scal;
+      vv[tid] = v;
+      A[tid * lda + r] = (tid == r) ? beta : v;
     }
-    if (tid == 0) {
-      vv[r] = T(1);
-      tau_out[r] = tau;
-    }
+    if (tid == 0) tau_out[r] = tau;
     __syncthreads();
-    if (tid == 0) A[r * lda + r] = beta;
-    if (r < min_dim - 1 && tau != T(0)) {
-      for (int c = r + 1 + tid; c < n; c += 512) {
-        T wsum = T(0);
-        for (int i = r; i < m; ++i) wsum += vv[i] * A[i * lda + c];
-        wsum *= tau;
-        for (int i = r; i < m; ++i) A[i * lda + c] -= wsum * vv[i];
+    // one pass: v^T A, for the columns of the block's reflectors V^T v
+    const bool later = col && c > r;
+    T ws = T(0);
+    if (tau != T(0) && (later || (c >= r0 && c < r))) ws = column_dot(r, vv);
+    if (c >= r0 && c < r) wk[c - r0] = ws;
+    __syncthreads();
+    bool anew = false;
+    if (later) {
+      T y = ws;
+#pragma unroll
+      for (int k = 0; k < B; ++k)
+        if (k < kb) y -= f[k] * wk[k];
+      y *= tau;
+      T rv = A[r * lda + c] - y;
+#pragma unroll
+      for (int k = 0; k < B; ++k) {
+        if (k < kb) rv -= vr[k] * f[k];
+        if (k == kb) f[k] = y;
       }
-    }
-    __syncthreads();
-    for (int c = r + 1 + tid; c < n; c += 512) {
-      if (cn[c] != T(0)) {
-        T temp = fabs(A[r * lda + c] / cn[c]);
+      A[r * lda + c] = rv;
+      if (cn != T(0)) {
+        T temp = fabs(rv / cn);
         temp = fmax(T(0), (T(1) - temp) * (T(1) + temp));
-        const T ratio = cn[c] / pcn[c];
+        const T ratio = cn / pcn;
         const T temp2 = temp * ratio * ratio;
         if (temp2 > tol3z) {
-          cn[c] = cn[c] * sqrt(temp);
+          cn = cn * sqrt(temp);
         } else if (r < m - 1) {
-          T s = T(0);
-          for (int i = r + 1; i < m; ++i) {
-            const T x = A[i * lda + c];
-            s += x * x;
-          }
-          cn[c] = sqrt(s);
-          pcn[c] = cn[c];
+          anew = true;
         } else {
-          cn[c] = T(0);
-          pcn[c] = T(0);
+          cn = T(0);
+          pcn = T(0);
         }
       }
     }
-    __syncthreads();
+    if (__syncthreads_or(anew)) {
+      T s = T(0);
+      updated_column(r + 1, r0, kb + 1, anew, [&](int, T x) { s += x * x; });
+      if (anew) {
+        cn = sqrt(s);
+        pcn = cn;
+      }
+    }
     ++r;
     if (r < n) {
       block_argmax(r, maxv, kmax);
     } else {
       maxv = T(0);
+      __syncthreads();
+    }
+    if (r - r0 == B && r < steps && (fixed || maxv > threshold)) {
+      // the tile up to date
+      updated_column(r, r0, B, col && c >= r, [&](int i, T x) { A[i * lda + c] = x; });
+#pragma unroll
+      for (int k = 0; k < B; ++k) f[k] = T(0);
+      r0 = r;
     }
   }
-  for (int c = tid; c < n; c += 512) it.piv[c] = piv[c];
+  if (col && c >= r) it.piv[c] = pc;
   if (tid == 0) *it.rank_out = (!fixed && !it.cap_trunc && r > it.cap) ? -r : r;
 }
 
