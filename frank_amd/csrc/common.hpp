@@ -244,6 +244,7 @@ struct Geqp3Item {
   void* tau;
   int32_t* piv;
   int32_t* rank_out;
+  int32_t* rank_copy;  // a second place for the rank, or null
   int32_t m, n, lda, cap;
   int32_t cap_trunc;  // stop after cap pivots instead of reporting the overflow
   int32_t pad;

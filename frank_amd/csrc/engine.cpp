@@ -92,8 +92,7 @@ Staging::~Staging() {
   if (d_) (void)hipFree(d_);
 }
 
-const void* Staging::push_bytes(const void* src, size_t bytes, hipStream_t s) {
-  const size_t aligned = (bytes + 255) & ~size_t(255);
+void Staging::room(size_t aligned, hipStream_t s) {
   if (off_ + aligned > cap_) {
     if (off_ != 0) {
       // the ring is in use by queued launches: drain before growing
@@ -110,6 +109,20 @@ const void* Staging::push_bytes(const void* src, size_t bytes, hipStream_t s) {
       cap_ = c;
     }
   }
+}
+
+void* Staging::readback(size_t bytes, void** dev, hipStream_t s) {
+  const size_t aligned = (bytes + 255) & ~size_t(255);
+  room(aligned, s);
+  *dev = hd_ + off_;
+  void* hp = h_ + off_;
+  off_ += aligned;
+  return hp;
+}
+
+const void* Staging::push_bytes(const void* src, size_t bytes, hipStream_t s) {
+  const size_t aligned = (bytes + 255) & ~size_t(255);
+  room(aligned, s);
   char* hp = h_ + off_;
   char* dp = d_ + off_;
   if (bytes) {
@@ -915,9 +928,12 @@ void compress_batched(const std::vector<CompressDesc<T>>& d, Context& ctx) {
     ctx.sync();
     ctx.reserve((size_t)nd * sizeof(T) * ((size_t)nmax + (size_t)mmax + (size_t)capmax * nmax * 2 + 4 * capmax +
                                             (size_t)capmax * capmax + 64) +
-                (size_t)nd * sizeof(int32_t) * (nmax + 64) + (size_t)16 * 4096);
+                (size_t)nd * sizeof(int32_t) * (nmax + 65) + (size_t)16 * 4096);
     T* tau = ctx.take<T>((size_t)nd * std::max(mmax, nmax));
     int32_t* piv = ctx.take<int32_t>((size_t)nd * nmax);
+    // the ranks also side by side: the tiles' own places are scattered, and a copy each
+    // (3 us, and the host in between) took as long as the factorization
+    int32_t* ranks = ctx.take<int32_t>((size_t)nd);
     std::vector<Geqp3Item> gi(nd);
     for (int t = 0; t < nd; ++t) {
       Geqp3Item g{};
@@ -925,6 +941,7 @@ void compress_batched(const std::vector<CompressDesc<T>>& d, Context& ctx) {
       g.tau = tau + (size_t)t * std::max(mmax, nmax);
       g.piv = piv + (size_t)t * nmax;
       g.rank_out = de[t].d_rank;
+      g.rank_copy = ranks + t;
       g.m = de[t].m;
       g.n = de[t].n;
       g.lda = (int)de[t].lda;
@@ -940,9 +957,11 @@ void compress_batched(const std::vector<CompressDesc<T>>& d, Context& ctx) {
       pl.run();
     }
     std::vector<int32_t> rk(nd);
-    for (int t = 0; t < nd; ++t)
-      FRK_HIP_CHECK(hipMemcpyAsync(&rk[t], de[t].d_rank, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    void* rdev;
+    const void* rhost = ctx.staging().readback(sizeof(int32_t) * ((size_t)nd + 1), &rdev, s);
+    launch_snapshot(static_cast<int32_t*>(rdev), ranks, nd, ranks, s);
     host_wait_stream(s, __func__);
+    std::memcpy(rk.data(), rhost, sizeof(int32_t) * nd);
     int rmax = 1;
     for (int t = 0; t < nd; ++t) {
       if (rk[t] < 0)
@@ -1301,15 +1320,18 @@ std::unique_ptr<BlrMatrix<T>> build_blr_kernel(const KernelDesc& kd, int nb_r, i
   for (int j = 0; j < nb_c; ++j) bmax = std::max<int64_t>(bmax, A->cols(j));
   const size_t per = (size_t)bmax * bmax;
   const int chunk = (int)std::max<int64_t>(1, std::min<int64_t>(1024, (int64_t(2) << 30) / (per * sizeof(T))));
-  DevBuf dense;
-  dense.ensure(sizeof(T) * per * std::min<size_t>(chunk, std::max<size_t>(lr.size(), 1)));
+  // the tiles before compression, at most 2 GiB (or one tile), kept with the context:
+  // builds that follow each other would have the driver hand out and clear as much
+  // again each time, which at 10 ms a build it does not keep up with
+  T* dense = static_cast<T*>(
+      ctx.persistent(8, sizeof(T) * per * std::min<size_t>(chunk, std::max<size_t>(lr.size(), 1))));
   for (size_t o = 0; o < lr.size(); o += chunk) {
     const size_t e = std::min(lr.size(), o + chunk);
     std::vector<GenItem> gl;
     std::vector<CompressDesc<T>> cd;
     for (size_t t = o; t < e; ++t) {
       const int i = lr[t].first, j = lr[t].second;
-      T* buf = dense.as<T>() + (t - o) * per;
+      T* buf = dense + (t - o) * per;
       GenItem g{};
       g.out = buf;
       g.ld = A->cols(j);

@@ -62,9 +62,13 @@ class Staging {
     return static_cast<const Item*>(push_bytes(v.data(), v.size() * sizeof(Item), s));
   }
   const void* push_bytes(const void* src, size_t bytes, hipStream_t s);
+  // A pinned slot for words a kernel writes (through `dev`) and the host reads once
+  // the stream has drained; valid until the next push or reset.
+  void* readback(size_t bytes, void** dev, hipStream_t s);
   void reset() { off_ = 0; }
 
  private:
+  void room(size_t aligned, hipStream_t s);
   char* h_ = nullptr;
   char* hd_ = nullptr;  // h_ as the device sees it
   char* d_ = nullptr;
@@ -141,7 +145,7 @@ class Context {
   // size allocates nothing.  Slots: 0, 1 refinement residual and correction;
   // 2, 3 tpmqrt's C copies and their ranks; 4 ranks of a typed batch's dense
   // compressions; 5 inverses of the batched tile LU; 6 tile-level tpqrt T;
-  // 7 partial sums of the kernel residual.
+  // 7 partial sums of the kernel residual; 8 tiles of a build before compression.
   void* persistent(int slot, size_t bytes) {
     DevBuf& b = persist_[slot];
     if (b.bytes() < bytes) {
@@ -185,7 +189,7 @@ class Context {
   hipEvent_t ev_open_ = nullptr;
   Context* owner_ = this;
   double peak_ = kPeakF64;
-  DevBuf persist_[8];
+  DevBuf persist_[9];
   hipStream_t aux_[2] = {nullptr, nullptr};
   void resolve_events();
 };

@@ -2347,6 +2347,7 @@ __global__ __launch_bounds__(512) void geqp3_kernel(const Geqp3Item* __restrict_
     if (tid == 0) {
       tau_out[0] = T(0);
       *it.rank_out = 1;
+      if (it.rank_copy) *it.rank_copy = 1;
     }
     return;
   }
@@ -2476,7 +2477,11 @@ __global__ __launch_bounds__(512) void geqp3_kernel(const Geqp3Item* __restrict_
     }
   }
   if (col && c >= r) it.piv[c] = pc;
-  if (tid == 0) *it.rank_out = (!fixed && !it.cap_trunc && r > it.cap) ? -r : r;
+  if (tid == 0) {
+    const int rk = (!fixed && !it.cap_trunc && r > it.cap) ? -r : r;
+    *it.rank_out = rk;
+    if (it.rank_copy) *it.rank_copy = rk;
+  }
 }
 
 template <typename T>
