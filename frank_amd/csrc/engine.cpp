@@ -2816,28 +2816,31 @@ void blr_matvec(BlrMatrix<T>& A, const T* x, T* y, int nrhs, Context& ctx) {
   for (int r : A.rank) kmax = std::max(kmax, r);
   ctx.reserve((size_t)nr * nc * 2 * sizeof(T) * ((size_t)kmax * nrhs + 64) + 4096);
   Plan pl(ctx);
+  // V x and S (V x) of every low-rank tile in a launch each; then y, a column of tiles
+  // at a time (the tiles of a row add to the same part of y, in column order)
+  std::vector<GemmItem> gv, gs;
+  std::vector<std::vector<GemmItem>> gy(nc);
   for (int j = 0; j < nc; ++j) {
-    std::vector<GemmItem> g1, g2, g3;
     const T* xj = x + A.coff[j] * nrhs;
     for (int i = 0; i < nr; ++i) {
       const int t = A.idx(i, j);
       T* yi = y + A.roff[i] * nrhs;
       const int mi = (int)A.rows(i), nj = (int)A.cols(j);
       if (A.kind[t] == kDense) {
-        g1.push_back(gemm_item(A.D[t], nj, 1, xj, nrhs, 1, yi, nrhs, 1, mi, nrhs, nj, 1.0, 1.0));
+        gy[j].push_back(gemm_item(A.D[t], nj, 1, xj, nrhs, 1, yi, nrhs, 1, mi, nrhs, nj, 1.0, 1.0));
       } else if (A.kind[t] == kLowRank) {
         const int r = A.rank[t];
         T* t1 = ctx.take<T>((size_t)r * nrhs + 1);
         T* t2 = ctx.take<T>((size_t)r * nrhs + 1);
-        g1.push_back(gemm_item(A.V[t], nj, 1, xj, nrhs, 1, t1, nrhs, 1, r, nrhs, nj, 1.0, 0.0));
-        g2.push_back(gemm_item(A.S[t], A.kcap, 1, t1, nrhs, 1, t2, nrhs, 1, r, nrhs, r, 1.0, 0.0));
-        g3.push_back(gemm_item(A.U[t], 1, mi, t2, nrhs, 1, yi, nrhs, 1, mi, nrhs, r, 1.0, 1.0));
+        gv.push_back(gemm_item(A.V[t], nj, 1, xj, nrhs, 1, t1, nrhs, 1, r, nrhs, nj, 1.0, 0.0));
+        gs.push_back(gemm_item(A.S[t], A.kcap, 1, t1, nrhs, 1, t2, nrhs, 1, r, nrhs, r, 1.0, 0.0));
+        gy[j].push_back(gemm_item(A.U[t], 1, mi, t2, nrhs, 1, yi, nrhs, 1, mi, nrhs, r, 1.0, 1.0));
       }
     }
-    plan_gemms<T>(pl, g1);
-    plan_gemms<T>(pl, g2);
-    plan_gemms<T>(pl, g3);
   }
+  plan_gemms<T>(pl, gv);
+  plan_gemms<T>(pl, gs);
+  for (const auto& g : gy) plan_gemms<T>(pl, g);
   pl.run();
 }
 
