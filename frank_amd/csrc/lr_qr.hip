@@ -55,7 +55,7 @@ struct Mma<double> {
   static __device__ __forceinline__ v4 mma(double a, double b, v4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
-  static constexpr double tiny = 1e-300;
+  static constexpr double tiny = 1e-300;  // of a column scaled to a largest entry in [1/2, 1)
 };
 template <>
 struct Mma<float> {
@@ -93,6 +93,26 @@ __device__ __forceinline__ double rows_sum(double v) {
   const auto l2 = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
   return __hiloint2double(h2[0], l2[0]) + __hiloint2double(h2[1], l2[1]);
 }
+// largest of the four lane rows' values (not NaN), in every lane
+__device__ __forceinline__ float rows_max(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+  v = fmaxf(__int_as_float(a[0]), __int_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+  return fmaxf(__int_as_float(b[0]), __int_as_float(b[1]));
+}
+__device__ __forceinline__ double rows_max(double v) {
+  const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+  const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+  v = fmax(__hiloint2double(h[0], l[0]), __hiloint2double(h[1], l[1]));
+  const auto h2 = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+  const auto l2 = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+  return fmax(__hiloint2double(h2[0], l2[0]), __hiloint2double(h2[1], l2[1]));
+}
+// e with |v| = f 2^e, f in [1/2, 1); 0 for zero, infinity and NaN.  x 2^e.
+__device__ __forceinline__ int exponent_of(double v) { return __builtin_amdgcn_frexp_exp(v); }
+__device__ __forceinline__ int exponent_of(float v) { return __builtin_amdgcn_frexp_expf(v); }
+__device__ __forceinline__ double scaled(double x, int e) { return __builtin_ldexp(x, e); }
+__device__ __forceinline__ float scaled(float x, int e) { return __builtin_ldexpf(x, e); }
 // v of lane row r (0..3), in every lane row
 template <int R>
 __device__ __forceinline__ int row_bcast(int v) {
@@ -213,7 +233,7 @@ __device__ __forceinline__ void qr_step(Panel<T, NT>& p, int li, int lr, int rw,
     }
   }
   const T q = bcast<J>(d), alpha = bcast<J>(xj);
-  const bool ok = q > M::tiny;  // a column of zeros is left as it is; a NaN in it stays one
+  const bool ok = q > M::tiny;  // a column of zeros (at its scale) is left as it is; a NaN in it stays one
   const T rn = rsqrt_of(q), nrm = q * rn;
   const T beta = (alpha >= T(0)) ? -nrm : nrm;
   const T den = fabs(alpha) + nrm, iden = inv_of(den);
@@ -441,6 +461,29 @@ __global__ __launch_bounds__(64 * NP * RW, (NT == 4 && NP == 8) ? 4 : 1) void lr
       if constexpr (RW > 1) __syncthreads();  // Wp free
     }
   }
+  // ---- every column to a largest entry in [1/2, 1), by a power of two ----------------
+  // Reflectors and T do not depend on the columns' scales, R takes them back: norms of
+  // any size neither overflow nor fall under `tiny`, which is then relative to the column.
+  int se = 0;
+  {
+    T mx = T(0);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mx = fmax(mx, fabs(x[t][e]));
+    mx = rows_max(mx);
+    if constexpr (RW > 1) {
+      if (lr == 0) Wp[256 * wid + li] = mx;
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < RW; ++r) mx = fmax(mx, Wp[256 * (w * RW + r) + li]);
+    }
+    se = exponent_of(mx);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[t][e] = scaled(x[t][e], -se);
+  }
   // ---- factorization, panel by panel ------------------------------------------------
   const Buf<T> Y(it.Y), Tg(it.tau);
   const int64_t ldy = it.y_cs;
@@ -486,7 +529,7 @@ __global__ __launch_bounds__(64 * NP * RW, (NT == 4 && NP == 8) ? 4 : 1) void lr
       for (int e = 0; e < 4; ++e) {
         const int row = 4 * lr + e;
         const T rv = (row < li) ? p.top[e] : (row == li ? p.rd : T(0));
-        Rb.store(at<T>(owner && own && j0 + row < K, kp + j0 + row, ldr, c, 1), (row < lim) ? rv : T(0));
+        Rb.store(at<T>(owner && own && j0 + row < K, kp + j0 + row, ldr, c, 1), (row < lim) ? scaled(rv, se) : T(0));
         p.top[e] = (li >= lim || row < li) ? T(0) : (row == li ? T(1) : p.top[e] * p.inv);
       }
 #pragma unroll
@@ -547,7 +590,7 @@ __global__ __launch_bounds__(64 * NP * RW, (NT == 4 && NP == 8) ? 4 : 1) void lr
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int row = j0 + 4 * lr + e;
-          Rb.store(at<T>(own && row < K, kp + row, ldr, c, 1), (row < nref) ? top[e] : T(0));
+          Rb.store(at<T>(own && row < K, kp + row, ldr, c, 1), (row < nref) ? scaled(top[e], se) : T(0));
         }
       }
     }
