@@ -92,6 +92,30 @@ __device__ __forceinline__ T wave_sum(T v) {
   v += xor16(v);
   return half_sum(v);
 }
+// e with |v| = f 2^e, f in [1/2, 1); 0 for zero, infinity and NaN.  x 2^e.
+__device__ __forceinline__ int exponent_of(double v) { return __builtin_amdgcn_frexp_exp(v); }
+__device__ __forceinline__ int exponent_of(float v) { return __builtin_amdgcn_frexp_expf(v); }
+__device__ __forceinline__ double scaled(double x, int e) { return __builtin_ldexp(x, e); }
+__device__ __forceinline__ float scaled(float x, int e) { return __builtin_ldexpf(x, e); }
+// largest of the 64 lanes' values (not NaN), in every lane
+__device__ __forceinline__ float half_max(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+  return fmaxf(__int_as_float(r[0]), __int_as_float(r[1]));
+}
+__device__ __forceinline__ double half_max(double v) {
+  const auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+  const auto l = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+  return fmax(__hiloint2double(h[0], l[0]), __hiloint2double(h[1], l[1]));
+}
+template <typename T>
+__device__ __forceinline__ T wave_max(T v) {
+  v = fmax(v, dpp_mov<0xB1>(v));
+  v = fmax(v, dpp_mov<0x4E>(v));
+  v = fmax(v, dpp_mov<0x141>(v));
+  v = fmax(v, dpp_mov<0x140>(v));
+  v = fmax(v, xor16(v));
+  return half_max(v);
+}
 
 // v of lane l (uniform l) in every lane
 __device__ __forceinline__ float wave_read(float v, int l) {
@@ -1051,6 +1075,24 @@ __global__ __launch_bounds__(W * 64) void qr_kernel(Src items) {
     }
   }
   const int kp = (it.P != nullptr) ? it.kp : 0;
+  // A column whose squares could leave the exponent range is scaled by a power of two
+  // (entries outside 2^-39 .. 2^39 in FP32: then the square of a remainder at rounding
+  // level, u times the entry, is still a normal number).  Reflectors do not depend on
+  // it, R takes it back.
+  int ex[CPW];
+  constexpr int kSafeExp = sizeof(T) == 8 ? 400 : 39;
+#pragma unroll
+  for (int q = 0; q < CPW; ++q) {
+    T mx = T(0);
+#pragma unroll
+    for (int t = 0; t < MR; ++t) mx = fmax(mx, fabs(a[q][t]));
+    ex[q] = __builtin_amdgcn_readfirstlane(exponent_of(wave_max(mx)));
+    if (ex[q] > -kSafeExp && ex[q] < kSafeExp) ex[q] = 0;
+    if (ex[q] != 0) {
+#pragma unroll
+      for (int t = 0; t < MR; ++t) a[q][t] = scaled(a[q][t], -ex[q]);
+    }
+  }
   // Step j = qj W + wj reflects column j, a[qj][] of wave wj: qj is unrolled, so the
   // column is addressed in registers directly (no selection over the array).
   static_assert(W * CPW <= 128, "row j < 128 lies in a[][0] or a[][1]");
@@ -1124,10 +1166,11 @@ __global__ __launch_bounds__(W * 64) void qr_kernel(Src items) {
       for (int t = 0; t < MR; ++t) {
         const int row = lane + 64 * t;
         if (row < m && row > c && c < nref) Y[row * it.y_rs + c * it.y_cs] = a[q][t];
+        const T rv = (ex[q] != 0) ? scaled(a[q][t], ex[q]) : a[q][t];
         if (it.r_upper_only) {
-          if (row <= c && row < nref) Rb[(int64_t)(kp + row) * ldr + c] = a[q][t];
+          if (row <= c && row < nref) Rb[(int64_t)(kp + row) * ldr + c] = rv;
         } else if (row < nref) {
-          Rb[(int64_t)(kp + row) * ldr + c] = (row <= c) ? a[q][t] : T(0);
+          Rb[(int64_t)(kp + row) * ldr + c] = (row <= c) ? rv : T(0);
         } else if (row < K) {
           Rb[(int64_t)(kp + row) * ldr + c] = T(0);
         }
@@ -1517,24 +1560,6 @@ void launch_tri_extract(const T* src, int64_t rs, int64_t cs, T* dst, int64_t ld
 // ===========================================================================
 // One-sided (Hestenes) Jacobi SVD of the K x K core with truncation.
 // ===========================================================================
-__device__ __forceinline__ float half_max(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
-  return fmaxf(__int_as_float(r[0]), __int_as_float(r[1]));
-}
-__device__ __forceinline__ double half_max(double v) {
-  const auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
-  const auto l = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
-  return fmax(__hiloint2double(h[0], l[0]), __hiloint2double(h[1], l[1]));
-}
-template <typename T>
-__device__ __forceinline__ T wave_max(T v) {
-  v = fmax(v, dpp_mov<0xB1>(v));
-  v = fmax(v, dpp_mov<0x4E>(v));
-  v = fmax(v, dpp_mov<0x141>(v));
-  v = fmax(v, dpp_mov<0x140>(v));
-  v = fmax(v, xor16(v));
-  return half_max(v);
-}
 // ---------------------------------------------------------------------------
 // LDS Jacobi SVD for K <= KMAX, one workgroup of KMAX / 2 groups of GL lanes per
 // core: group g serves columns g and g + KMAX / 2 (QR phase), or the column pair
