@@ -742,7 +742,7 @@ void plan_lr_add(Plan& pl, const std::vector<LrAddDesc<T>>& d_in, int lra) {
     reach(x.kx1, x.xs_ld, x.kx2, 1);
     reach(x.kx2, x.xv_rs, x.n, x.xv_cs);
   }
-  if (near && lr_blocked_ok<T>(nd, std::max(mmax, nmax), std::max(qk, capmax))) {
+  if (sizeof(T) == 8 && near && lr_blocked_ok(nd, std::max(mmax, nmax), std::max(qk, capmax))) {
     b.Kp = (K + 15) / 16 * 16;
     b.ldu = (mmax + 15) / 16 * 16;
     b.ldv = (nmax + 15) / 16 * 16;

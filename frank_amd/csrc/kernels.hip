@@ -2211,10 +2211,9 @@ void launch_svd(const SvdItem* d_items, int n_items, int max_k, hipStream_t s) {
 
 template <typename T>
 void launch_lr_add_qr(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, int max_k, hipStream_t s) {
-  if (b.Kp > 0)
-    launch_lr_qr_blocked<T>(d, nd, b, max_k, s);
-  else
-    launch_qr_src<T>(LrQrItems<T>{d, b}, 2 * nd, max_k, s, std::max(b.mmax, b.nmax));
+  if constexpr (sizeof(T) == 8)
+    if (b.Kp > 0) return launch_lr_qr_blocked(d, nd, b, max_k, s);
+  launch_qr_src<T>(LrQrItems<T>{d, b}, 2 * nd, max_k, s, std::max(b.mmax, b.nmax));
 }
 template <typename T>
 void launch_lr_add_svd(const LrAddDesc<T>* d, int t0, int n, int max_k, const LrBatch<T>& b, hipStream_t s) {
@@ -2222,10 +2221,9 @@ void launch_lr_add_svd(const LrAddDesc<T>* d, int t0, int n, int max_k, const Lr
 }
 template <typename T>
 void launch_lr_add_apply(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, int max_ncol, hipStream_t s) {
-  if (b.Kp > 0)
-    launch_lr_apply_blocked<T>(d, nd, b, max_ncol, s);
-  else
-    launch_apply_q_src<T>(LrApplyItems<T>{d, b}, 2 * nd, max_ncol, s, std::max(b.mmax, b.nmax));
+  if constexpr (sizeof(T) == 8)
+    if (b.Kp > 0) return launch_lr_apply_blocked(d, nd, b, max_ncol, s);
+  launch_apply_q_src<T>(LrApplyItems<T>{d, b}, 2 * nd, max_ncol, s, std::max(b.mmax, b.nmax));
 }
 
 // ===========================================================================

@@ -119,14 +119,11 @@ void launch_rows_scatter(const RowRef* d_rows, int R, const T* W, int N, hipStre
 // the core, basis update), items derived on the device from the descriptors.
 template <typename T>
 void launch_lr_add_qr(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, int max_k, hipStream_t s);
-// The blocked forms (lr_qr.hip) of the QR and the basis update: whether they are used
-// for nd additions of up to m rows and k columns, and their launches (b.Kp > 0).
-template <typename T>
+// The blocked forms (lr_qr.hip) of the QR and the basis update in FP64: whether they are
+// used for nd additions of up to m rows and k columns, and their launches (b.Kp > 0).
 bool lr_blocked_ok(int nd, int m, int k);
-template <typename T>
-void launch_lr_qr_blocked(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, int k, hipStream_t s);
-template <typename T>
-void launch_lr_apply_blocked(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, int k, hipStream_t s);
+void launch_lr_qr_blocked(const LrAddDesc<double>* d, int nd, const LrBatch<double>& b, int k, hipStream_t s);
+void launch_lr_apply_blocked(const LrAddDesc<double>* d, int nd, const LrBatch<double>& b, int k, hipStream_t s);
 template <typename T>
 void launch_lr_add_core(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, hipStream_t s);
 template <typename T>

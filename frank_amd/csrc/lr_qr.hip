@@ -1,4 +1,5 @@
-// Blocked QR and basis update of the batched low-rank additions (gfx950).
+// Blocked QR and basis update of the batched FP64 low-rank additions, and the core
+// product of additions with more columns than rows (gfx950).
 //
 // QR of a panel [A1 S1 | A2 S2] (m x K): a wave holds 16 of the columns in registers,
 // as NT tiles of 16 x 16 in the layout of an MFMA result: lane (j, r), j = lane & 15,
@@ -21,6 +22,9 @@
 // products, a reduction, rsq and rcp with their corrections, the update; with the
 // exchange between two waves 1200) and the update of the next panel's columns; in
 // large batches by FP64 issue (MFMA and vector units have the same FP64 rate).
+// FP64 only: in FP32 the compact WY form (T, and one more rounding of T^T W) left an
+// error of the sum of 2.2e-7 at m = 256, K = 32, singular values 10^(-i/2), against
+// 1.8e-7 with a reflector at a time, which the additions in FP32 keep.
 // Measured, FP64, QR of both panels and basis update, us, these kernels / the
 // unblocked ones (a reflector at a time over the whole panel, two barriers each):
 //   m    K    additions   QR             update
@@ -55,7 +59,6 @@ struct Mma<double> {
   static __device__ __forceinline__ v4 mma(double a, double b, v4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
-  static constexpr double tiny = 1e-300;  // of a column scaled to a largest entry in [1/2, 1)
 };
 template <>
 struct Mma<float> {
@@ -66,7 +69,6 @@ struct Mma<float> {
   static __device__ __forceinline__ v4 mma(float a, float b, v4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
-  static constexpr float tiny = 1e-36f;
 };
 
 // lane J of the 16-lane row, in every lane of the row
@@ -74,17 +76,7 @@ template <int J>
 __device__ __forceinline__ double bcast(double v) {
   return __builtin_amdgcn_update_dpp(0.0, v, 0x150 + J, 0xF, 0xF, true);
 }
-template <int J>
-__device__ __forceinline__ float bcast(float v) {
-  return __builtin_amdgcn_update_dpp(0.0f, v, 0x150 + J, 0xF, 0xF, true);
-}
 // sum over the four lane rows, in every lane
-__device__ __forceinline__ float rows_sum(float v) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
-  v = __int_as_float(a[0]) + __int_as_float(a[1]);
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
-  return __int_as_float(b[0]) + __int_as_float(b[1]);
-}
 __device__ __forceinline__ double rows_sum(double v) {
   const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
   const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
@@ -94,12 +86,6 @@ __device__ __forceinline__ double rows_sum(double v) {
   return __hiloint2double(h2[0], l2[0]) + __hiloint2double(h2[1], l2[1]);
 }
 // largest of the four lane rows' values (not NaN), in every lane
-__device__ __forceinline__ float rows_max(float v) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
-  v = fmaxf(__int_as_float(a[0]), __int_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
-  return fmaxf(__int_as_float(b[0]), __int_as_float(b[1]));
-}
 __device__ __forceinline__ double rows_max(double v) {
   const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
   const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
@@ -110,9 +96,7 @@ __device__ __forceinline__ double rows_max(double v) {
 }
 // e with |v| = f 2^e, f in [1/2, 1); 0 for zero, infinity and NaN.  x 2^e.
 __device__ __forceinline__ int exponent_of(double v) { return __builtin_amdgcn_frexp_exp(v); }
-__device__ __forceinline__ int exponent_of(float v) { return __builtin_amdgcn_frexp_expf(v); }
 __device__ __forceinline__ double scaled(double x, int e) { return __builtin_ldexp(x, e); }
-__device__ __forceinline__ float scaled(float x, int e) { return __builtin_ldexpf(x, e); }
 // v of lane row r (0..3), in every lane row
 template <int R>
 __device__ __forceinline__ int row_bcast(int v) {
@@ -122,10 +106,6 @@ __device__ __forceinline__ int row_bcast(int v) {
   return b[R >> 1];
 }
 template <int R>
-__device__ __forceinline__ float row_bcast(float v) {
-  return __int_as_float(row_bcast<R>(__float_as_int(v)));
-}
-template <int R>
 __device__ __forceinline__ double row_bcast(double v) {
   return __hiloint2double(row_bcast<R>(__double2hiint(v)), row_bcast<R>(__double2loint(v)));
 }
@@ -133,57 +113,51 @@ __device__ __forceinline__ double row_bcast(double v) {
 // element (the compiler makes a broadcast copy and a multiply-add).  The leading
 // s_nop covers a DPP source written by the instruction before the block, which the
 // compiler does not see; results of matrix instructions pass mma_fence() first.
-#define FRK_FMAC_DPP4(TY, O0, O1, O2, O3, A0, A1, A2, A3, B0, B1, B2, B3, IMM)        \
-  "s_nop 1\n\t"                                                                       \
-  "v_fmac_" TY "_dpp " O0 ", " A0 ", " B0 " row_newbcast:" IMM " row_mask:0xf bank_mask:0xf\n\t" \
-  "v_fmac_" TY "_dpp " O1 ", " A1 ", " B1 " row_newbcast:" IMM " row_mask:0xf bank_mask:0xf\n\t" \
-  "v_fmac_" TY "_dpp " O2 ", " A2 ", " B2 " row_newbcast:" IMM " row_mask:0xf bank_mask:0xf\n\t" \
-  "v_fmac_" TY "_dpp " O3 ", " A3 ", " B3 " row_newbcast:" IMM " row_mask:0xf bank_mask:0xf"
-#define FRK_DPP_PAIR(T, TY)                                                                            \
-  template <int J>                                                                                     \
-  __device__ __forceinline__ void dot4(T& s0, T& s1, T& s2, T& s3, T x0, T x1, T x2, T x3) {           \
-    asm(FRK_FMAC_DPP4(TY, "%0", "%1", "%2", "%3", "%4", "%5", "%6", "%7", "%4", "%5", "%6", "%7", "%8") \
-        : "+v"(s0), "+v"(s1), "+v"(s2), "+v"(s3)                                                       \
-        : "v"(x0), "v"(x1), "v"(x2), "v"(x3), "n"(J));                                                 \
-  }                                                                                                    \
-  template <int J>                                                                                     \
-  __device__ __forceinline__ void axpy4(T& x0, T& x1, T& x2, T& x3, T w) {                             \
-    asm(FRK_FMAC_DPP4(TY, "%0", "%1", "%2", "%3", "%0", "%1", "%2", "%3", "%4", "%4", "%4", "%4", "%5") \
-        : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3)                                                       \
-        : "v"(w), "n"(J));                                                                             \
-  }                                                                                                    \
-  /* a0 += g(K) t0 + g(K+2) t2, a1 likewise: g(k) lane k's value */                                   \
-  template <int K>                                                                                     \
-  __device__ __forceinline__ void tdot4(T& a0, T& a1, T g, T t0, T t1, T t2, T t3) {                   \
-    asm("s_nop 1\n\t"                                                                                  \
-        "v_fmac_" TY "_dpp %0, %2, %3 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"                  \
-        "v_fmac_" TY "_dpp %1, %2, %4 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"                  \
-        "v_fmac_" TY "_dpp %0, %2, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"                  \
-        "v_fmac_" TY "_dpp %1, %2, %6 row_newbcast:%10 row_mask:0xf bank_mask:0xf"                      \
-        : "+v"(a0), "+v"(a1)                                                                           \
-        : "v"(g), "v"(t0), "v"(t1), "v"(t2), "v"(t3), "n"(K), "n"(K + 1), "n"(K + 2), "n"(K + 3));     \
-  }                                                                                                    \
-  /* waits until a matrix instruction's result may be read by the blocks above */                      \
-  __device__ __forceinline__ void mma_fence(T& x0, T& x1, T& x2, T& x3) {                              \
-    asm volatile("s_nop 15\n\ts_nop 7" : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3));                      \
-  }
-FRK_DPP_PAIR(double, "f64")
-FRK_DPP_PAIR(float, "f32")
+#define FRK_FMAC_DPP4(O0, O1, O2, O3, A0, A1, A2, A3, B0, B1, B2, B3, IMM)              \
+  "s_nop 1\n\t"                                                                         \
+  "v_fmac_f64_dpp " O0 ", " A0 ", " B0 " row_newbcast:" IMM " row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f64_dpp " O1 ", " A1 ", " B1 " row_newbcast:" IMM " row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f64_dpp " O2 ", " A2 ", " B2 " row_newbcast:" IMM " row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f64_dpp " O3 ", " A3 ", " B3 " row_newbcast:" IMM " row_mask:0xf bank_mask:0xf"
+template <int J>
+__device__ __forceinline__ void dot4(double& s0, double& s1, double& s2, double& s3, double x0, double x1, double x2,
+                                     double x3) {
+  asm(FRK_FMAC_DPP4("%0", "%1", "%2", "%3", "%4", "%5", "%6", "%7", "%4", "%5", "%6", "%7", "%8")
+      : "+v"(s0), "+v"(s1), "+v"(s2), "+v"(s3)
+      : "v"(x0), "v"(x1), "v"(x2), "v"(x3), "n"(J));
+}
+template <int J>
+__device__ __forceinline__ void axpy4(double& x0, double& x1, double& x2, double& x3, double w) {
+  asm(FRK_FMAC_DPP4("%0", "%1", "%2", "%3", "%0", "%1", "%2", "%3", "%4", "%4", "%4", "%4", "%5")
+      : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3)
+      : "v"(w), "n"(J));
+}
+// a0 += g(K) t0 + g(K+2) t2, a1 likewise: g(k) lane k's value
+template <int K>
+__device__ __forceinline__ void tdot4(double& a0, double& a1, double g, double t0, double t1, double t2, double t3) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %2, %3 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %2, %4 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %2, %6 row_newbcast:%10 row_mask:0xf bank_mask:0xf"
+      : "+v"(a0), "+v"(a1)
+      : "v"(g), "v"(t0), "v"(t1), "v"(t2), "v"(t3), "n"(K), "n"(K + 1), "n"(K + 2), "n"(K + 3));
+}
+// waits until a matrix instruction's result may be read by the blocks above
+__device__ __forceinline__ void mma_fence(double& x0, double& x1, double& x2, double& x3) {
+  asm volatile("s_nop 15\n\ts_nop 7" : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3));
+}
 // 1 / sqrt(x) and 1 / x to about an ulp, without branches (x = 0 gives NaN or inf)
 __device__ __forceinline__ double rsqrt_of(double x) {
   const double r = __builtin_amdgcn_rsq(x);
   const double e = fma(-x * r, r, 1.0);
   return fma(r * e, fma(0.375, e, 0.5), r);
 }
-__device__ __forceinline__ float rsqrt_of(float x) {
-  const float r = __builtin_amdgcn_rsqf(x);
-  return fmaf(0.5f * r, fmaf(-x * r, r, 1.0f), r);
-}
 __device__ __forceinline__ double inv_of(double x) { return d64::rcp2(x); }
-__device__ __forceinline__ float inv_of(float x) {
-  const float r = __builtin_amdgcn_rcpf(x);
-  return fmaf(fmaf(-x, r, 1.0f), r, r);
-}
+
+// Squared norm at and below which a pivot column counts as zero, of a column scaled to
+// a largest entry in [1/2, 1).
+constexpr double kZeroNorm2 = 1e-300;
 
 // A wave's share of a panel: tiles x (tile t is tile t RW + rw of the column), the
 // pivot rows' tile (taken out of x; zero in a wave that does not own it), row li of
@@ -233,7 +207,7 @@ __device__ __forceinline__ void qr_step(Panel<T, NT>& p, int li, int lr, int rw,
     }
   }
   const T q = bcast<J>(d), alpha = bcast<J>(xj);
-  const bool ok = q > M::tiny;  // a column of zeros (at its scale) is left as it is; a NaN in it stays one
+  const bool ok = q > kZeroNorm2;  // a column of zeros (at its scale) is left as it is; a NaN in it stays one
   const T rn = rsqrt_of(q), nrm = q * rn;
   const T beta = (alpha >= T(0)) ? -nrm : nrm;
   const T den = fabs(alpha) + nrm, iden = inv_of(den);
@@ -767,7 +741,6 @@ void apply_go(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, hipStream_t s)
 // used most (m = 512, K up to 32, several hundred additions, ranks below 16: 138 us a
 // launch in a factorization of 64 x 64 tiles, the blocked form with four waves a
 // panel 185).
-template <typename T>
 bool lr_blocked_ok(int nd, int m, int k) {
   return k <= 128 && (m <= 128 || (m <= 256 && (k > 32 || nd <= 128)));
 }
@@ -785,14 +758,13 @@ bool lr_blocked_ok(int nd, int m, int k) {
       FN(8);            \
   } while (0)
 
-template <typename T>
-void launch_lr_qr_blocked(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, int k, hipStream_t s) {
+void launch_lr_qr_blocked(const LrAddDesc<double>* d, int nd, const LrBatch<double>& b, int k, hipStream_t s) {
   if (nd <= 0) return;
   const int m = std::max(b.mmax, b.nmax);
   if (m > 256 || k > 128 || b.Kp <= 0) throw std::runtime_error("lr qr: panel outside the blocked kernels");
-#define FRK_QR4(NP) qr_go<T, 4, 1, NP>(d, nd, b, s)
-#define FRK_QR8(NP) qr_go<T, 8, 1, NP>(d, nd, b, s)
-#define FRK_QR16(NP) qr_go<T, (NP) < 8 ? 8 : 16, (NP) < 8 ? 2 : 1, NP>(d, nd, b, s)
+#define FRK_QR4(NP) qr_go<double, 4, 1, NP>(d, nd, b, s)
+#define FRK_QR8(NP) qr_go<double, 8, 1, NP>(d, nd, b, s)
+#define FRK_QR16(NP) qr_go<double, (NP) < 8 ? 8 : 16, (NP) < 8 ? 2 : 1, NP>(d, nd, b, s)
   if (m <= 64)
     FRK_LR_COLS(FRK_QR4);
   else if (m <= 128)
@@ -804,14 +776,13 @@ void launch_lr_qr_blocked(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, in
 #undef FRK_QR16
   FRK_HIP_CHECK(hipGetLastError());
 }
-template <typename T>
-void launch_lr_apply_blocked(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, int k, hipStream_t s) {
+void launch_lr_apply_blocked(const LrAddDesc<double>* d, int nd, const LrBatch<double>& b, int k, hipStream_t s) {
   if (nd <= 0) return;
   const int m = std::max(b.mmax, b.nmax);
   if (m > 256 || k > 128 || b.Kp <= 0) throw std::runtime_error("lr apply: panel outside the blocked kernels");
-#define FRK_AP4(NW) apply_go<T, 4, 1, NW>(d, nd, b, s)
-#define FRK_AP8(NW) apply_go<T, 8, 1, NW>(d, nd, b, s)
-#define FRK_AP16(NW) apply_go<T, (NW) < 8 ? 8 : 16, (NW) < 8 ? 2 : 1, NW>(d, nd, b, s)
+#define FRK_AP4(NW) apply_go<double, 4, 1, NW>(d, nd, b, s)
+#define FRK_AP8(NW) apply_go<double, 8, 1, NW>(d, nd, b, s)
+#define FRK_AP16(NW) apply_go<double, (NW) < 8 ? 8 : 16, (NW) < 8 ? 2 : 1, NW>(d, nd, b, s)
   if (m <= 64)
     FRK_LR_COLS(FRK_AP4);
   else if (m <= 128)
@@ -835,12 +806,7 @@ void launch_lr_add_core(const LrAddDesc<T>* d, int nd, const LrBatch<T>& b, hipS
   FRK_HIP_CHECK(hipGetLastError());
 }
 
-#define FRK_LRQR_INST(T)                                                                                   \
-  template bool lr_blocked_ok<T>(int, int, int);                                                                \
-  template void launch_lr_qr_blocked<T>(const LrAddDesc<T>*, int, const LrBatch<T>&, int, hipStream_t);    \
-  template void launch_lr_apply_blocked<T>(const LrAddDesc<T>*, int, const LrBatch<T>&, int, hipStream_t); \
-  template void launch_lr_add_core<T>(const LrAddDesc<T>*, int, const LrBatch<T>&, hipStream_t);
-FRK_LRQR_INST(double)
-FRK_LRQR_INST(float)
+template void launch_lr_add_core<double>(const LrAddDesc<double>*, int, const LrBatch<double>&, hipStream_t);
+template void launch_lr_add_core<float>(const LrAddDesc<float>*, int, const LrBatch<float>&, hipStream_t);
 
 }  // namespace frk
