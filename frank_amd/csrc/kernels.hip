@@ -1569,10 +1569,13 @@ void launch_tri_extract(const T* src, int64_t rs, int64_t cs, T* dst, int64_t ld
 //      [1, 2): exact, and squared norms stay clear of underflow).
 //   2. Column-pivoted Householder QR, M P = Q R, in registers: every wave offers
 //      its best remaining column through LDS, so a step costs one barrier.  It
-//      stops once the trailing block is below delta = max(u, 1e-3 eps) ||M||_F
-//      (u: the unit roundoff, eps: the truncation accuracy): the block enters the
-//      kept singular values in second order only (sigma^2 moves by at most
-//      delta^2), and the rotations then run on rp < K columns.
+//      stops at the numerical rank rp, once the trailing block E is below the floor
+//      at which the rotations take a column for zero (u ||M||_F, u the unit
+//      roundoff, or less for a smaller eps).  Stopping earlier, at a share of the
+//      truncation accuracy, would leave the sum U S V alone but move the kept
+//      singular values, by ||E||^2 / 2 sigma.  VG goes on to the end: it takes
+//      u = M v / sigma, in which E v / sigma remains (stopping at u ||M||_F, U^T U
+//      was off by 1.7e-5 instead of 9.0e-6 at sigma_r = 1e-8 ||M||).
 //   3. One-sided Jacobi on R^T (K x rp), whose graded rows converge in few sweeps
 //      (Drmac-Veselic), a round-robin schedule, one barrier a round.  The
 //      rotations also turn Q into the left vectors.  VG (FP64, K > 64: the second
@@ -1823,12 +1826,9 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   // rounding noise.  The floor also stays a factor 16 under the truncation
   // threshold eps ||sigma|| / sqrt(K) of an eps-rank decision, so in FP32 at eps
   // near 1e-6 the columns the rank is decided on are still rotated.
-  T fl = Eps<T>::v, fd = Eps<T>::v;
-  if (it.fixed_rank < 0 && it.eps > 0.0) {
-    fl = fmin(fl, static_cast<T>(it.eps / (16.0 * sqrt((double)K))));
-    fd = fmax(fl, static_cast<T>(1e-3 * it.eps));
-  }
-  const T tiny = fl * fl * fro2, delta2 = fd * fd * fro2;
+  T fl = Eps<T>::v;
+  if (it.fixed_rank < 0 && it.eps > 0.0) fl = fmin(fl, static_cast<T>(it.eps / (16.0 * sqrt((double)K))));
+  const T tiny = fl * fl * fro2, delta2 = VG ? T(0) : tiny;
   // ---- 2. pivoted QR, columns in registers -----------------------------------
   bool live0 = c0 < K, live1 = c1 < K;
   int rp = 0;

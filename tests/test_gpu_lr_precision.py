@@ -48,3 +48,36 @@ def test_fp32_sums(torch_gpu, fa, m):
     err = [(_norm(D - U @ (S @ V)) - np.linalg.norm(t)) / _norm(D) for (U, S, V), D, t in zip(out, Ds, tails)]
     print(f"fp32 sums m={m}: mean error {np.mean(err):.3e}", flush=True)
     assert np.mean(err) <= 4.0 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("eps", [1e-2, 1e-4, 1e-6, 1e-8])
+@pytest.mark.parametrize("k", [6, 8, 16, 32, 64])
+@pytest.mark.parametrize("decay", [0.1, 0.5])
+def test_parts_of_a_truncated_sum(torch_gpu, fa, k, eps, decay):
+    """The singular values and bases that a truncation keeps are those of the whole sum, to rounding, and
+    not only the product U S V within eps."""
+    rng = np.random.default_rng(k)
+    u = np.finfo(np.float64).eps
+    out, Ds = _add(torch_gpu, fa, [_operands(rng, 200, 150, k, k, decay) for _ in range(8)], "float64", eps,
+                   "rounded_addition")
+    for (U, S, V), D in zip(out, Ds):
+        r, K = U.shape[1], 2 * k
+        sv = np.linalg.svd(D.astype(np.float64), compute_uv=False)
+        # each side (K reflectors, the core's rotations; numpy's own) to a few sqrt(K) u of the norm
+        assert np.abs(np.diag(S).astype(np.float64) - sv[:r]).max() <= 8 * np.sqrt(K) * u * np.linalg.norm(sv)
+        # vectors orthogonal to the rotation threshold tol = 8 max(K, 8) u; above 64 columns u_i = M v_i / sigma_i,
+        # in which the larger ones stand with sigma_j (v_j^T v_i) / sigma_i
+        tol = 8 * max(K, 8) * u
+        assert np.abs((V @ V.T).astype(np.float64) - np.eye(r)).max() <= 2 * tol
+        assert np.abs((U.T @ U).astype(np.float64) - np.eye(r)).max() <= 2 * tol * (sv[0] / sv[r - 1] if K > 64 else 1)
+
+
+def test_left_vectors_of_large_cores(torch_gpu, fa):
+    """Above 64 columns, sigma_r = 1e-8 of the norm: orthogonal to 9.0e-6 in the mean of 48 additions with
+    the core's QR run to its end, to 1.7e-5 when it stops at u ||M||_F and 2.8e-5 at 1e-11 ||M||_F."""
+    rng = np.random.default_rng(7)
+    out, _ = _add(torch_gpu, fa, [_operands(rng, 200, 150, 64, 64, 0.5) for _ in range(48)], "float64", 1e-8,
+                  "rounded_addition")
+    err = [np.abs((U.T @ U).astype(np.float64) - np.eye(U.shape[1])).max() for U, _, _ in out]
+    print(f"left vectors: {np.mean(err):.3e}", flush=True)
+    assert np.mean(err) <= 1.3e-5

@@ -69,8 +69,9 @@ def test_tile_edges(torch_gpu, fa, dtype, lra, case):
         assert tail <= (eps + 8 * K * u) * np.linalg.norm(sv) or eps == 0.0
         # products of K reflectors times vectors orthogonal to the rotation threshold 8 max(K, 8) u
         assert np.abs(V @ V.T - np.eye(r)).max() <= 16 * max(K, 8) * u
-        if not (dtype == "float64" and K > 64):  # that core forms u = M v / sigma: ||M|| / sigma_r times u
-            assert np.abs(U.T @ U - np.eye(r)).max() <= 16 * max(K, 8) * u
+        # above 64 columns FP64 forms u_i = M v_i / sigma_i: the same times sigma_1 / sigma_r
+        lim = 16 * max(K, 8) * u * (sv[0] / sv[r - 1] if dtype == "float64" and K > 64 else 1.0)
+        assert np.abs(U.T @ U - np.eye(r)).max() <= lim
 
 
 @pytest.mark.parametrize("dtype", ["float64", "float32"])

@@ -60,8 +60,9 @@ def test_core_sizes(torch_gpu, fa, dtype, k1, k2, decay):
         assert np.abs(np.diag(S) - sv[:r]).max() <= 8 * K * u * sv[0]
         # right vectors: pairwise orthogonal to the rotation threshold 8 max(K, 8) u
         assert np.abs(V @ V.T - np.eye(r)).max() <= 16 * max(K, 8) * u
-        if not (dtype == "float64" and K > 64):  # that variant forms u = M v / sigma: ||M|| / sigma_r times u
-            assert np.abs(U.T @ U - np.eye(r)).max() <= 16 * max(K, 8) * u
+        # above 64 columns FP64 forms u_i = M v_i / sigma_i: the same times sigma_1 / sigma_r
+        lim = 16 * max(K, 8) * u * (sv[0] / sv[r - 1] if dtype == "float64" and K > 64 else 1.0)
+        assert np.abs(U.T @ U - np.eye(r)).max() <= lim
         # the oracle's rank, where the decision is not within rounding of the threshold
         want = fo.find_svd_truncation_rank(sv[:min(K, len(sv))], eps)
         if dtype == "float64":
