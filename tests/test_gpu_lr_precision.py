@@ -81,3 +81,25 @@ def test_left_vectors_of_large_cores(torch_gpu, fa):
     err = [np.abs((U.T @ U).astype(np.float64) - np.eye(U.shape[1])).max() for U, _, _ in out]
     print(f"left vectors: {np.mean(err):.3e}", flush=True)
     assert np.mean(err) <= 1.3e-5
+
+
+@pytest.mark.parametrize("m,n,k1,k2", [(64, 60, 5, 3), (64, 64, 16, 9), (128, 100, 17, 16), (256, 200, 16, 16),
+                                       (256, 256, 40, 24)])
+def test_projection_leaves_nothing_of_the_basis(torch_gpu, fa, m, n, k1, k2):
+    """The fast addition projects X's bases on C's.  Where X lies within 1e-7 of them and that remainder
+    decides what is kept, the new basis is still orthonormal to rounding."""
+    rng = np.random.default_rng(m + k1)
+    u = np.finfo(np.float64).eps
+    ops = []
+    for _ in range(4):
+        A = _operands(rng, m, n, k1, k1, 0.0)[0]
+        k = min(k1, k2)
+        near = lambda W: np.linalg.qr(W[:, rng.permutation(k1)[:k]] + 1e-7 * rng.standard_normal((W.shape[0], k)))[0]
+        U, V = near(A[0]), near(A[2].T)
+        # X = U V^T at 1e14: what it has outside C's bases, 1e-7 of each, weighs as much as C itself
+        ops.append(((A[0], A[1], A[2]), (U, 1e14 * np.eye(k), V.T)))
+    out, _ = _add(torch_gpu, fa, ops, "float64", 0.0, "fast_rounded_addition")
+    for U, S, V in out:
+        K = k1 + k2
+        assert np.abs((U.T @ U).astype(np.float64) - np.eye(U.shape[1])).max() <= 16 * max(K, 8) * u
+        assert np.abs((V @ V.T).astype(np.float64) - np.eye(U.shape[1])).max() <= 16 * max(K, 8) * u
