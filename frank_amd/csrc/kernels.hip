@@ -1682,6 +1682,11 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   using vec = typename LdsVec<T, VW>::type;
   const SvdItem it = items.get(blockIdx.x);
   const int K = it.K;
+  // the core of up to 16 columns (FP64: 32) is taken transposed: G's vectors, orthogonal to
+  // the rotation threshold (5e-14 at K = 32), are then the left ones, and the right ones are
+  // products of reflectors and rotations (5e-15).  The fixed-rank block LU loses less that
+  // way round (1.25 times at 16 x 16 tiles of 256, rank 16, geometric mean of 12 matrices).
+  constexpr bool TR = KMAX <= 16 || (KMAX <= 32 && sizeof(T) == 8);
   __shared__ __align__(16) T G[KMAX * LD];
   __shared__ __align__(16) T Vs[VG ? VW : KMAX * LD];  // reflectors, then Q, then the left vectors
   __shared__ T taus[KMAX], sig[KMAX], sigs[KMAX], coef[KMAX];
@@ -1727,18 +1732,19 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   for (int e = 0; e < RL; ++e) x0[e] = x1[e] = T(0);
   if (it.mode == 0) {
     const T* M = static_cast<const T*>(it.M);
+    const int64_t rs = TR ? it.m_cs : it.m_rs, cs = TR ? it.m_rs : it.m_cs;
 #pragma unroll
     for (int e = 0; e < RL; ++e) {
       const int row = row_of(e);
-      if (row < K && c0 < K) x0[e] = M[row * it.m_rs + c0 * it.m_cs];
-      if (row < K && c1 < K) x1[e] = M[row * it.m_rs + c1 * it.m_cs];
+      if (row < K && c0 < K) x0[e] = M[row * rs + c0 * cs];
+      if (row < K && c1 < K) x1[e] = M[row * rs + c1 * cs];
     }
   } else {
     // M(i, j) = sum_t Ru(i, t) Rv(j, t): Ru (and Rv when there is room) staged by
     // columns; Ru and Rv are upper triangular below their first ka rows
     const int J = it.kx;
-    const T* Ru = static_cast<const T*>(it.Ru);
-    const T* Rv = static_cast<const T*>(it.Rv);
+    const T* Ru = static_cast<const T*>(TR ? it.Rv : it.Ru);
+    const T* Rv = static_cast<const T*>(TR ? it.Ru : it.Rv);
     for (int e = tid; e < KMAX * J; e += NT) {
       const int i = e / J, t = e - (e / J) * J;
       G[t * LD + i] = (i < K) ? Ru[i * it.ldr + t] : T(0);
@@ -1776,11 +1782,12 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
     }
     if (it.ka > 0) {
       const T* Sa = static_cast<const T*>(it.Sa);
+      const int rs = TR ? 1 : it.lds_in, cs = TR ? it.lds_in : 1;
 #pragma unroll
       for (int e = 0; e < RL; ++e) {
         const int row = row_of(e);
-        if (row < it.ka && c0 < it.ka) x0[e] += Sa[row * it.lds_in + c0];
-        if (row < it.ka && c1 < it.ka) x1[e] += Sa[row * it.lds_in + c1];
+        if (row < it.ka && c0 < it.ka) x0[e] += Sa[row * rs + c0 * cs];
+        if (row < it.ka && c1 < it.ka) x1[e] += Sa[row * rs + c1 * cs];
       }
     }
   }
@@ -2136,8 +2143,9 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
     }
   }
   T* S = static_cast<T*>(it.S);
-  T* Um = static_cast<T*>(it.Um);
-  T* Vm = static_cast<T*>(it.Vm);
+  T* Um = static_cast<T*>(TR ? it.Vm : it.Um);
+  T* Vm = static_cast<T*>(TR ? it.Um : it.Vm);
+  const int ldu = TR ? it.ldv : it.ldu, ldv = TR ? it.ldu : it.ldv;
   if (S != nullptr)
     for (int e = tid; e < r * r; e += NT) {
       const int i = e / r, j = e - (e / r) * r;
@@ -2145,9 +2153,9 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
     }
   for (int e = tid; e < K * r; e += NT) {
     const int row = e / r, c = e - (e / r) * r;
-    if (Vm != nullptr) Vm[row * it.ldv + c] = G[order[c] * LD + row];
+    if (Vm != nullptr) Vm[row * ldv + c] = G[order[c] * LD + row];
     if constexpr (!VG) {
-      if (Um != nullptr) Um[row * it.ldu + c] = Vs[order[c] * LD + row];
+      if (Um != nullptr) Um[row * ldu + c] = Vs[order[c] * LD + row];
     }
   }
   if constexpr (VG) {
@@ -2170,7 +2178,7 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
             const int row = i0 + 4 * v + lk;
-            if (row < K) Um[row * it.ldu + c] = (sc > sig_floor) ? acc[v] / sc : T(0);
+            if (row < K) Um[row * ldu + c] = (sc > sig_floor) ? acc[v] / sc : T(0);
           }
         }
       }

@@ -103,3 +103,21 @@ def test_projection_leaves_nothing_of_the_basis(torch_gpu, fa, m, n, k1, k2):
         K = k1 + k2
         assert np.abs((U.T @ U).astype(np.float64) - np.eye(U.shape[1])).max() <= 16 * max(K, 8) * u
         assert np.abs((V @ V.T).astype(np.float64) - np.eye(U.shape[1])).max() <= 16 * max(K, 8) * u
+
+
+@pytest.mark.parametrize("lra,eps", [("rounded_addition", 0.0), ("rounded_addition", 1e-10), ("fast_rounded_addition", 0.0)])
+@pytest.mark.parametrize("k", [4, 8, 12, 16])
+def test_right_vectors_of_small_cores(torch_gpu, fa, k, lra, eps):
+    """Up to 32 columns in FP64 the right vectors come from reflectors and rotations alone: orthogonal to
+    a few roundings a reflector, 2 K u, below the rotation threshold of 8 max(K, 8) u (the left ones')."""
+    rng = np.random.default_rng(k)
+    u = np.finfo(np.float64).eps
+    out, Ds = _add(torch_gpu, fa, [_operands(rng, 128, 100, k, k, d) for d in (0.1, 0.3, 0.5) for _ in range(8)],
+                   "float64", eps, lra)
+    K = 2 * k
+    for (U, S, V), D in zip(out, Ds):
+        r = U.shape[1]
+        assert np.abs((V @ V.T).astype(np.float64) - np.eye(r)).max() <= 2 * K * u
+        assert np.abs((U.T @ U).astype(np.float64) - np.eye(r)).max() <= 16 * max(K, 8) * u
+        tail = np.linalg.norm(np.linalg.svd(D.astype(np.float64), compute_uv=False)[r:])
+        assert _norm(D - U @ (S @ V)) <= tail * (1 + 1e-6) + 8 * K * u * _norm(D)
