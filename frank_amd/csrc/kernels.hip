@@ -1603,9 +1603,7 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
   return fma(r * e, fma(0.375, e, 0.5), r);
 }
 __device__ __forceinline__ double sqrt_nr(double x) { return x > 0.0 ? x * rsqrt_nr(x) : x; }
-__device__ __forceinline__ float sqrt_nr(float x) { return sqrtf(x); }
 __device__ __forceinline__ double inv_nr(double x) { return d64::rcp2(x); }
-__device__ __forceinline__ float inv_nr(float x) { return 1.0f / x; }
 // Rotation (c, s) that zeroes the off-diagonal of [[al, ga], [ga, be]].  FP64:
 // cos 2t = |d| / h and sin 2t = 2 ga / h with d = be - al, h = sqrt(d^2 + 4 ga^2):
 // two reciprocal square roots, no division (the squares cannot underflow, since
@@ -1672,6 +1670,28 @@ __device__ __forceinline__ T dot_tree(const T (&x)[N], const T (&y)[N]) {
   return p[0];
 }
 
+// sum_e x[e]^2 in FP64.  Squared norms of FP32 columns are kept so: what a pivot column's
+// norm is off by goes into R's diagonal whole, and what tau is off by makes its
+// reflector that much less orthogonal.
+template <int N>
+__device__ __forceinline__ double norm2(const double (&x)[N]) {
+  return dot_tree(x, x);
+}
+template <int N>
+__device__ __forceinline__ double norm2(const float (&x)[N]) {
+  double y[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) y[k] = x[k];
+  return dot_tree(y, y);
+}
+// tau = 2 / w^T w of the reflector w = x - beta e, from q = x^T x and w's entry at e
+__device__ __forceinline__ double tau_of(double q, double alpha, double beta, double) {
+  return inv_nr(q - alpha * beta);
+}
+__device__ __forceinline__ float tau_of(double q, float alpha, float, float we) {
+  return (float)(2.0 * inv_nr(fma((double)we, (double)we, fma(-(double)alpha, (double)alpha, q))));
+}
+
 template <typename T, int KMAX, int GL, bool VG, class Src>
 __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   constexpr int NG = KMAX / 2, NT = NG * GL, NW = NT / 64, RL = KMAX / GL;
@@ -1690,7 +1710,8 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   __shared__ __align__(16) T G[KMAX * LD];
   __shared__ __align__(16) T Vs[VG ? VW : KMAX * LD];  // reflectors, then Q, then the left vectors
   __shared__ T taus[KMAX], sig[KMAX], sigs[KMAX], coef[KMAX];
-  __shared__ T candq[2][NW], wmax[NW];
+  __shared__ double candq[2][NW];
+  __shared__ T wmax[NW];
   __shared__ unsigned candk[2][NW];
   __shared__ int order[KMAX];
   __shared__ int rank_sh, lastrot_sh, accept_sh;
@@ -1808,7 +1829,7 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
     x0[e] *= scale;
     x1[e] *= scale;
   }
-  T q0 = group_sum(dot_tree(x0, x0), GL), q1 = group_sum(dot_tree(x1, x1), GL);
+  double q0 = group_sum(norm2(x0), GL), q1 = group_sum(norm2(x1), GL);
   if (sub == 0) {
     sig[c0] = q0;
     sig[c1] = q1;
@@ -1859,15 +1880,15 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
     const unsigned ka = lanes_umax<NW>(candk[buf][lane % NW]);
     const int pv = 127 - (int)(ka & 0x7Fu);
     const int pw = ((pv >= NG ? pv - NG : pv) * GL) >> 6;
-    const T q = candq[buf][pw];
-    if (q * T(K - rp) <= delta2) break;
+    const double q = candq[buf][pw];
+    if (q * (K - rp) <= delta2) break;
     const T* pc = G + (buf * NW + pw) * LD;
     T v[RL];
     load_col(pc, v);
     const T alpha = pc[rp];
-    const T nrm = sqrt_nr(q);
+    const T nrm = (T)sqrt_nr(q);
     const T beta = (alpha >= T(0)) ? -nrm : nrm;
-    const T tau = inv_nr(q - alpha * beta);  // H = I - tau w w^T, w = x - beta e
+    const T tau = tau_of(q, alpha, beta, alpha - beta);  // H = I - tau w w^T, w = x - beta e
 #pragma unroll
     for (int e = 0; e < RL; ++e) {
       const int row = row_of(e);
@@ -1894,8 +1915,8 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
       z0[e] = (row > rp) ? x0[e] : T(0);
       z1[e] = (row > rp) ? x1[e] : T(0);
     }
-    q0 = group_sum(dot_tree(z0, z0), GL);
-    q1 = group_sum(dot_tree(z1, z1), GL);
+    q0 = group_sum(norm2(z0), GL);
+    q1 = group_sum(norm2(z1), GL);
   }
   const int n = rp;
   __syncthreads();  // the last candidates are read, the reflectors complete
@@ -2001,9 +2022,9 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   // ---- singular values, their order, the rank ----------------------------------
   load_col(G + c0 * LD, x0);
   load_col(G + c1 * LD, x1);
-  q0 = group_sum(dot_tree(x0, x0), GL);
-  q1 = group_sum(dot_tree(x1, x1), GL);
-  const T s0 = (c0 < n) ? sqrt(q0) : T(0), s1 = (c1 < n) ? sqrt(q1) : T(0);
+  q0 = group_sum(norm2(x0), GL);
+  q1 = group_sum(norm2(x1), GL);
+  const T s0 = (c0 < n) ? (T)sqrt(q0) : T(0), s1 = (c1 < n) ? (T)sqrt(q1) : T(0);
   if (sub == 0) {
     sig[c0] = s0;
     sig[c1] = s1;

@@ -50,6 +50,19 @@ def test_fp32_sums(torch_gpu, fa, m):
     assert np.mean(err) <= 4.0 * 2.0 ** -24
 
 
+@pytest.mark.parametrize("m,limit", [(64, 1.95e-7), (512, 1.7e-7)])
+def test_fp32_cores(torch_gpu, fa, m, limit):
+    """The same mean with the squared column norms of the core's QR in FP64: 1.81e-7 at m = 64 and 1.59e-7
+    at m = 512; with them in FP32 2.09 and 1.80e-7.  The limits lie between."""
+    rng = np.random.default_rng(m)
+    out, Ds = _add(torch_gpu, fa, [_operands(rng, m, m, 16, 16, 0.5) for _ in range(48)], "float32", 1e-6,
+                   "rounded_addition")
+    tails = [np.linalg.svd(D.astype(np.float64), compute_uv=False)[U.shape[1]:] for (U, _, _), D in zip(out, Ds)]
+    err = [(_norm(D - U @ (S @ V)) - np.linalg.norm(t)) / _norm(D) for (U, S, V), D, t in zip(out, Ds, tails)]
+    print(f"fp32 cores m={m}: mean error {np.mean(err):.3e}", flush=True)
+    assert np.mean(err) <= limit
+
+
 @pytest.mark.parametrize("eps", [1e-2, 1e-4, 1e-6, 1e-8])
 @pytest.mark.parametrize("k", [6, 8, 16, 32, 64])
 @pytest.mark.parametrize("decay", [0.1, 0.5])
