@@ -1856,7 +1856,9 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   // near 1e-6 the columns the rank is decided on are still rotated.
   T fl = Eps<T>::v;
   if (it.fixed_rank < 0 && it.eps > 0.0) fl = fmin(fl, static_cast<T>(it.eps / (16.0 * sqrt((double)K))));
-  const T tiny = fl * fl * fro2, delta2 = VG ? T(0) : tiny;
+  // (an infinity in M makes fro2 one: nothing is small against it, and what it meets
+  // becomes NaN)
+  const T tiny = fl * fl * fro2, delta2 = (VG || !isfinite(fro2)) ? T(0) : tiny;
   // ---- 2. pivoted QR, columns in registers -----------------------------------
   bool live0 = c0 < K, live1 = c1 < K;
   int rp = 0;
@@ -2030,6 +2032,8 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
     sig[c1] = s1;
     order[c0] = c0;
     order[c1] = c1;
+    sigs[c0] = s0;  // (NaN has no place in the order: what nothing else claims stays)
+    sigs[c1] = s1;
   }
   __syncthreads();
   {
@@ -2117,7 +2121,7 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   T thr = T(0.25);
   for (int c = 0; c < r; ++c) {
     const int src = order[c];
-    if (sigs[c] > sig_floor) continue;
+    if (!(sigs[c] <= sig_floor)) continue;  // (NaN stays as it is)
     for (int tries = 0; tries < 2 * K; ++tries, --u) {
       if (u < 0) {
         u = K - 1;

@@ -87,3 +87,32 @@ def test_fixed_rank_above_the_numerical_rank(torch_gpu, fa, dtype, k1, k2):
         assert np.linalg.norm(D - (U @ S) @ V) <= 8 * K * u * np.linalg.norm(D)
         assert np.abs(V @ V.T - np.eye(k1)).max() <= 16 * max(K, 8) * u
         assert np.abs(U.T @ U - np.eye(k1)).max() <= 16 * max(K, 8) * u
+
+
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("k", [4, 8, 16, 32, 64])
+@pytest.mark.parametrize("kind", ["overflow", "inf", "nan"])
+def test_core_that_is_not_finite(torch_gpu, fa, dtype, k, kind):
+    """A core that overflows (bases of a large norm), or operands with an infinity or a NaN, give a tile
+    that is not finite either, and not zeros; the other additions of the batch are not touched."""
+    print(f"not finite {dtype} K={2 * k} {kind}", flush=True)
+    torch = torch_gpu
+    rng = np.random.default_rng(k)
+    u = np.finfo(dtype).eps
+    A, B = _pair(rng, 150, 140, k, k, 0.1, False)
+    bad = [x.copy() for x in A]
+    if kind == "overflow":
+        big = 1e30 if dtype == "float32" else 1e200
+        bad[1] = big * bad[1]
+        bad[2] = big * bad[2]
+    else:
+        bad[0][3, 1] = np.inf if kind == "inf" else np.nan
+    for eps in (1e-5, 0.0):
+        X, Y, Z = _add(torch, fa, [(A, B), (tuple(bad), B), (A, B)], 128, eps, getattr(torch, dtype))
+        assert not np.isfinite((Y[0] @ Y[1]) @ Y[2]).any()
+        for x, z in zip(X, Z):
+            assert np.array_equal(x, z)
+        D = (A[0] @ A[1]) @ A[2] + (B[0] @ B[1]) @ B[2]
+        sv = np.linalg.svd(D, compute_uv=False)
+        tail = np.linalg.norm(sv[X[0].shape[1]:])
+        assert np.linalg.norm(D - (X[0] @ X[1]) @ X[2]) <= tail * (1 + 1e-5) + 16 * k * u * np.linalg.norm(sv)
