@@ -2012,7 +2012,7 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
       if (rounds - lastrot_sh >= n2 - 1 || rounds >= 60 * (n2 - 1)) break;
     }
   }
-  const int sweeps = (rounds + n2 - 2) / max(1, n2 - 1);
+  const int sweeps = (n < 2) ? 0 : (rounds + n2 - 2) / (n2 - 1);
   if (tid == 0 && it.stats != nullptr) {
     // this workgroup's copy of the counters (a line of its own: no contention
     // between the items of a launch)

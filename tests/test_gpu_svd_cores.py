@@ -116,3 +116,27 @@ def test_core_that_is_not_finite(torch_gpu, fa, dtype, k, kind):
         sv = np.linalg.svd(D, compute_uv=False)
         tail = np.linalg.norm(sv[X[0].shape[1]:])
         assert np.linalg.norm(D - (X[0] @ X[1]) @ X[2]) <= tail * (1 + 1e-5) + 16 * k * u * np.linalg.norm(sv)
+
+
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+def test_sweep_counters_with_zero_cores(torch_gpu, fa, dtype):
+    """Zero cores and cores of one column count as problems of no sweeps."""
+    torch = torch_gpu
+    rng = np.random.default_rng(1)
+    dt = getattr(torch, dtype)
+    ctx = fa.Context()
+    for k, scale, most in ((8, 0.0, 0), (32, 0.0, 0), (8, 1.0, 60)):
+        pairs = [_pair(rng, 90, 80, k, k, 0.1, False) for _ in range(5)]
+        As, Bs = [], []
+        for (U, S, V), B in pairs:
+            slots = [torch.zeros(s, dtype=dt, device="cuda") for s in ((90, 64), (64, 64), (64, 80))]
+            for t, x in zip(slots, (U, scale * S, V)):
+                t[:x.shape[0], :x.shape[1]] = torch.from_numpy(np.ascontiguousarray(x)).to("cuda", dt)
+            As.append((*slots, k))
+            Bs.append(tuple(torch.from_numpy(np.ascontiguousarray(x)).to("cuda", dt) for x in (B[0], scale * B[1], B[2])))
+        ctx.counters(reset=True)
+        fa.lr_add_batched(As, Bs, eps=0.0, lra="rounded_addition", cap=64, ctx=ctx)
+        c = ctx.counters()
+        assert c["svd_problems"] == 5
+        assert (0 if scale == 0.0 else 5) <= c["svd_sweeps"] <= 5 * most
+        assert 0 <= c["svd_max_sweeps"] <= most
