@@ -1606,14 +1606,19 @@ __device__ __forceinline__ double sqrt_nr(double x) { return x > 0.0 ? x * rsqrt
 __device__ __forceinline__ double inv_nr(double x) { return d64::rcp2(x); }
 // Rotation (c, s) that zeroes the off-diagonal of [[al, ga], [ga, be]].  FP64:
 // cos 2t = |d| / h and sin 2t = 2 ga / h with d = be - al, h = sqrt(d^2 + 4 ga^2):
-// two reciprocal square roots, no division (the squares cannot underflow, since
-// al and be exceed (u ||M||_F)^2 after the scaling).  FP32, whose squares could:
+// two reciprocal square roots, no division (at a tiny eps the floor of al and be lies
+// so low that their squares underflow: d and ga are scaled up then).  FP32:
 // Rutishauser's formulas, t = sign(zeta) / (|zeta| + sqrt(1 + zeta^2)), zeta =
 // (be - al) / (2 ga), c = 1 / sqrt(1 + t^2), s = c t, on the hardware reciprocal
 // and roots (about 1 ulp: only the angle moves, the rotation stays orthogonal).
 __device__ __forceinline__ void jacobi_rotation(double al, double be, double ga, double& c, double& s) {
-  const double d = be - al;
-  const double w = rsqrt_nr(fma(d, d, 4.0 * ga * ga));
+  double d = be - al, h2 = fma(d, d, 4.0 * ga * ga);
+  if (h2 < 1e-280) {
+    d = ldexp(d, 600);
+    ga = ldexp(ga, 600);
+    h2 = fma(d, d, 4.0 * ga * ga);
+  }
+  const double w = rsqrt_nr(h2);
   const double c2 = fma(0.5 * fabs(d), w, 0.5);
   const double rc = rsqrt_nr(c2);
   c = c2 * rc;
@@ -1864,10 +1869,10 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   int rp = 0;
   for (; rp < K; ++rp) {
     const int buf = rp & 1;
-    // the remaining column of largest norm: the norm's leading float bits above
-    // the column index (the smaller index on a tie)
-    const unsigned k0 = live0 ? ((__float_as_uint((float)q0) & ~0x7Fu) | (unsigned)(127 - c0)) : 0u;
-    const unsigned k1 = live1 ? ((__float_as_uint((float)q1) & ~0x7Fu) | (unsigned)(127 - c1)) : 0u;
+    // the remaining column of largest norm: the squared norm's leading bits (exponent
+    // and 13 of the fraction) above the column index (the smaller index on a tie)
+    const unsigned k0 = live0 ? (((unsigned)__double2hiint(q0) & ~0x7Fu) | (unsigned)(127 - c0)) : 0u;
+    const unsigned k1 = live1 ? (((unsigned)__double2hiint(q1) & ~0x7Fu) | (unsigned)(127 - c1)) : 0u;
     const unsigned kg = umax32(k0, k1), kw = groups_umax<GL>(kg);
     if (kg == kw && (live0 || live1)) {
       const bool first = k0 == kw && live0;

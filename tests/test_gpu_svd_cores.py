@@ -140,3 +140,24 @@ def test_sweep_counters_with_zero_cores(torch_gpu, fa, dtype):
         assert c["svd_problems"] == 5
         assert (0 if scale == 0.0 else 5) <= c["svd_sweeps"] <= 5 * most
         assert 0 <= c["svd_max_sweeps"] <= most
+
+
+@pytest.mark.parametrize("k", [4, 8, 16, 32])
+@pytest.mark.parametrize("low", [1e-30, 1e-85, 1e-120])
+def test_blocks_of_very_different_norm(torch_gpu, fa, k, low):
+    """A tile and `low` times another on other rows and columns, at an eps below that ratio: nothing mixes
+    them, so the small one is kept, and as accurately as the large one."""
+    print(f"blocks K={2 * k} {low:g}", flush=True)
+    rng = np.random.default_rng(k)
+    u = np.finfo(float).eps
+    parts, tiles = [], []
+    for rows, cols, scale in ((slice(0, 80), slice(0, 70), 1.0), (slice(80, 150), slice(70, 130), low)):
+        # (bases that are not orthonormal: the cores then need rotations)
+        X, Y = rng.standard_normal((rows.stop - rows.start, k)), rng.standard_normal((k, cols.stop - cols.start))
+        U, V = np.zeros((150, k)), np.zeros((k, 130))
+        U[rows], V[:, cols] = X, Y
+        parts.append((U, scale * np.eye(k), V))
+        tiles.append((rows, cols, scale, X @ Y))
+    ((U, S, V),) = _add(torch_gpu, fa, [tuple(parts)], 128, 1e-3 * low, torch_gpu.float64)
+    for rows, cols, scale, D in tiles:
+        assert np.linalg.norm((U[rows] @ (S / scale)) @ V[:, cols] - D) <= 8 * 2 * k * u * np.linalg.norm(D)
