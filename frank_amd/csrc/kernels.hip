@@ -1828,11 +1828,11 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   for (int w = 1; w < NW; ++w) amax = fmax(amax, wmax[w]);
   int sexp = 0;
   if (amax > T(0) && isfinite(amax)) sexp = ilogb(amax);
-  const T scale = ldexp(T(1), -sexp), unscale = ldexp(T(1), sexp);
+  // (entry by entry: 2^-sexp itself is no number where M is denormal)
 #pragma unroll
   for (int e = 0; e < RL; ++e) {
-    x0[e] *= scale;
-    x1[e] *= scale;
+    x0[e] = scaled(x0[e], -sexp);
+    x1[e] = scaled(x1[e], -sexp);
   }
   double q0 = group_sum(norm2(x0), GL), q1 = group_sum(norm2(x1), GL);
   if (sub == 0) {
@@ -2179,7 +2179,7 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   if (S != nullptr)
     for (int e = tid; e < r * r; e += NT) {
       const int i = e / r, j = e - (e / r) * r;
-      S[i * it.lds + j] = (i == j) ? sigs[i] * unscale : T(0);
+      S[i * it.lds + j] = (i == j) ? scaled(sigs[i], sexp) : T(0);
     }
   for (int e = tid; e < K * r; e += NT) {
     const int row = e / r, c = e - (e / r) * r;

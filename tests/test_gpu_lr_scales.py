@@ -73,3 +73,26 @@ def test_columns_of_different_norms_and_zero_columns(torch_gpu, fa, dtype):
         D = (A[0] @ A[1]) @ A[2] + (B[0] @ B[1]) @ B[2]
         U, S, V = (x.double().cpu().numpy() for x in (U[:, :r], S[:r, :r], V[:r]))
         assert np.linalg.norm(D - (U @ S) @ V) <= (1.01e-5 + 16 * k * u) * np.linalg.norm(D)
+
+
+@pytest.mark.parametrize("dtype,scale", [("float32", 2.0 ** -132), ("float64", 2.0 ** -1030)])
+@pytest.mark.parametrize("k", [6, 12, 24, 40])
+def test_denormal_tiles(torch_gpu, fa, dtype, scale, k):
+    """A tile of denormal numbers is recompressed to their spacing."""
+    torch = torch_gpu
+    rng = np.random.default_rng(k)
+    u, dt, cap, m, n = np.finfo(dtype).eps, getattr(torch, dtype), 128, 120, 100
+    spacing = float(np.finfo(dtype).smallest_subnormal) / scale  # in the operands' own units
+    up = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to("cuda", dt)
+    A, B = _pair(rng, m, n, k, k)
+    A, B = (A[0], np.eye(k), A[2]), (B[0], np.eye(k), B[2])
+    U, S, V = (torch.zeros(s, dtype=dt, device="cuda") for s in ((m, cap), (cap, cap), (cap, n)))
+    U[:, :k], S[:k, :k], V[:k] = up(A[0]), up(scale * A[1]), up(A[2])
+    (r,) = fa.lr_add_batched([(U, S, V, k)], [(up(B[0]), up(scale * B[1]), up(B[2]))], eps=1e-3,
+                             lra="rounded_addition", cap=cap)
+    D = A[0] @ A[2] + B[0] @ B[2]
+    U, S, V = (x.double().cpu().numpy() for x in (U[:, :r], S[:r, :r], V[:r]))
+    K = 2 * k
+    # both panels' entries and the core's are rounded to the spacing (m K, K^2 of them, taken through K products)
+    lim = (1.01e-3 + 8 * K * u) * np.linalg.norm(D) + spacing * K * np.sqrt(m * n)
+    assert np.linalg.norm(D - (U @ (S / scale)) @ V) <= lim
