@@ -1,5 +1,6 @@
 // Host orchestration of the batched BLR operations (see engine.hpp).
 #include "engine.hpp"
+#include "near.hpp"
 #include "plan.hpp"
 
 #include <algorithm>
@@ -728,20 +729,7 @@ void plan_lr_add(Plan& pl, const std::vector<LrAddDesc<T>>& d_in, int lra) {
   }
   LrBatch<T> b{};
   // the blocked QR and basis update address an operand with 31-bit byte offsets
-  bool near = true;
-  auto reach = [&](int64_t r, int64_t rs, int64_t c, int64_t cs) {
-    if (r <= 0 || c <= 0) return;
-    constexpr int64_t lim = (int64_t)0x7fffff00 / (int64_t)sizeof(T);
-    near = near && rs >= 0 && cs >= 0 && rs < lim && cs < lim && (r - 1) * rs + (c - 1) * cs < lim;
-  };
-  for (const auto& x : d) {
-    reach(x.m, x.cu_rs, x.kc, x.cu_cs);
-    reach(x.kc, x.cv_rs, x.n, x.cv_cs);
-    reach(x.kc, x.lds, x.kc, 1);
-    reach(x.m, x.xu_rs, x.kx1, x.xu_cs);
-    reach(x.kx1, x.xs_ld, x.kx2, 1);
-    reach(x.kx2, x.xv_rs, x.n, x.xv_cs);
-  }
+  const bool near = std::all_of(d.begin(), d.end(), [](const LrAddDesc<T>& x) { return near_addition<T>(x); });
   if (sizeof(T) == 8 && near && lr_blocked_ok(nd, std::max(mmax, nmax), std::max(qk, capmax))) {
     b.Kp = (K + 15) / 16 * 16;
     b.ldu = (mmax + 15) / 16 * 16;
