@@ -48,6 +48,7 @@ _SIGS = {
     "frk_ctx_create": ([C.POINTER(vp)], C.c_int),
     "frk_ctx_destroy": ([vp], C.c_int),
     "frk_ctx_synchronize": ([vp], C.c_int),
+    "frk_ctx_trim": ([vp], C.c_int),
     "frk_blr_create_kernel": ([vp, C.c_int, C.c_int, i64, vp, dbl, dbl, C.c_int, dbl, C.c_int, dbl, C.c_int,
                                C.c_int, C.c_int, C.POINTER(vp)], C.c_int),
     "frk_blr_create": ([vp, C.c_int, C.c_int, vp, vp, vp, C.c_int, dbl, C.c_int, C.c_int, C.POINTER(vp)], C.c_int),

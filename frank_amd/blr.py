@@ -50,6 +50,11 @@ class Context:
     def synchronize(self):
         L.check(L.lib().frk_ctx_synchronize(self.h))
 
+    def trim(self):
+        """Give the workspace and the scratch buffers that the context keeps between calls
+        (up to 2 GiB after a build) back to the driver; the next call allocates what it needs."""
+        L.check(L.lib().frk_ctx_trim(self.h))
+
     @property
     def stream_ptr(self) -> int:
         p = C.c_void_p()

@@ -228,6 +228,14 @@ int frk_ctx_synchronize(frk_ctx ctx) {
   });
 }
 
+int frk_ctx_trim(frk_ctx ctx) {
+  return guard([&] {
+    if (!ctx) throw std::invalid_argument("ctx is null");
+    ctx->ctx->trim();
+    return FRK_OK;
+  });
+}
+
 int frk_ctx_stream(frk_ctx ctx, void** stream) {
   return guard([&] {
     if (!ctx || !stream) throw std::invalid_argument("null argument");

@@ -69,6 +69,12 @@ DevBuf::~DevBuf() {
   if (p_) (void)hipFree(p_);
 }
 
+void DevBuf::release() {
+  if (p_) FRK_HIP_CHECK(hipFree(p_));
+  p_ = nullptr;
+  bytes_ = 0;
+}
+
 void DevBuf::ensure(size_t bytes) {
   if (bytes <= bytes_) return;
   if (p_) FRK_HIP_CHECK(hipFree(p_));
@@ -199,6 +205,14 @@ void Context::sync() {
   stage_.reset();
   ws_off_ = 0;
   resolve_events();
+}
+
+void Context::trim() {
+  for (hipStream_t a : aux_)
+    if (a) host_wait_stream(a, __func__);
+  sync();
+  ws_.release();
+  for (DevBuf& b : persist_) b.release();
 }
 
 void Context::account(const char* cls, double flops, double bytes, double peak, int64_t launches) {
@@ -1308,9 +1322,11 @@ std::unique_ptr<BlrMatrix<T>> build_blr_kernel(const KernelDesc& kd, int nb_r, i
   for (int j = 0; j < nb_c; ++j) bmax = std::max<int64_t>(bmax, A->cols(j));
   const size_t per = (size_t)bmax * bmax;
   const int chunk = (int)std::max<int64_t>(1, std::min<int64_t>(1024, (int64_t(2) << 30) / (per * sizeof(T))));
-  // the tiles before compression, at most 2 GiB (or one tile), kept with the context:
-  // builds that follow each other would have the driver hand out and clear as much
-  // again each time, which at 10 ms a build it does not keep up with
+  // the tiles before compression, at most 2 GiB (or one tile), kept with the context until
+  // trim(): builds that follow each other would have the driver hand out and clear as much
+  // again each time, which at 10 ms a build it does not keep up with.  Fewer tiles at a
+  // time leave compute units idle: N = 16384 (32 x 32 tiles of 512) 6.9 ms, 7.3 at 1 GiB,
+  // 7.9 at 512 MiB, 11.8 at 256; N = 32768 25.8, 29.9, 33.6 and 49.5 ms.
   T* dense = static_cast<T*>(
       ctx.persistent(8, sizeof(T) * per * std::min<size_t>(chunk, std::max<size_t>(lr.size(), 1))));
   for (size_t o = 0; o < lr.size(); o += chunk) {

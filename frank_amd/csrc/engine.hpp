@@ -41,6 +41,7 @@ class DevBuf {
     o.bytes_ = 0;
   }
   void ensure(size_t bytes);  // grows; contents are not preserved
+  void release();
   template <class X>
   X* as() const {
     return static_cast<X*>(p_);
@@ -109,6 +110,7 @@ class Context {
   void* take_bytes(size_t bytes);
   void reset_ws() { ws_off_ = 0; }
   void sync();  // drain the stream, reset staging and workspace
+  void trim();  // sync(), and free the workspace and the persistent buffers
   // identity matrix (ident_n x ident_n) in both precisions
   template <class X>
   const X* identity(int n);

@@ -67,6 +67,12 @@ int frk_version(void);
 int frk_ctx_create(frk_ctx* out);
 int frk_ctx_destroy(frk_ctx ctx);
 int frk_ctx_synchronize(frk_ctx ctx);
+
+/* Give the device memory that ctx keeps between calls back to the driver: its
+ * workspace and its scratch buffers, among them the tiles of a matrix build before
+ * compression (up to 2 GiB).  Drains the stream; matrices are not touched, and the
+ * next call that needs a buffer allocates it anew. */
+int frk_ctx_trim(frk_ctx ctx);
 /* The hipStream_t every call on this context is ordered on (for events / interop). */
 int frk_ctx_stream(frk_ctx ctx, void** stream);
 /* Device event counters of this context (no reference counterpart; the
