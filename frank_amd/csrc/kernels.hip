@@ -1573,9 +1573,7 @@ void launch_tri_extract(const T* src, int64_t rs, int64_t cs, T* dst, int64_t ld
 //      at which the rotations take a column for zero (u ||M||_F, u the unit
 //      roundoff, or less for a smaller eps).  Stopping earlier, at a share of the
 //      truncation accuracy, would leave the sum U S V alone but move the kept
-//      singular values, by ||E||^2 / 2 sigma.  VG goes on to the end: it takes
-//      u = M v / sigma, in which E v / sigma remains (stopping at u ||M||_F, U^T U
-//      was off by 1.7e-5 instead of 9.0e-6 at sigma_r = 1e-8 ||M||).
+//      singular values, by ||E||^2 / 2 sigma.
 //   3. One-sided Jacobi on R^T (K x rp), whose graded rows converge in few sweeps
 //      (Drmac-Veselic), a round-robin schedule, one barrier a round.  The
 //      rotations also turn Q into the left vectors.  VG (FP64, K > 64: the second
@@ -1863,7 +1861,7 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   if (it.fixed_rank < 0 && it.eps > 0.0) fl = fmin(fl, static_cast<T>(it.eps / (16.0 * sqrt((double)K))));
   // (an infinity in M makes fro2 one: nothing is small against it, and what it meets
   // becomes NaN)
-  const T tiny = fl * fl * fro2, delta2 = (VG || !isfinite(fro2)) ? T(0) : tiny;
+  const T tiny = fl * fl * fro2, delta2 = !isfinite(fro2) ? T(0) : tiny;
   // ---- 2. pivoted QR, columns in registers -----------------------------------
   bool live0 = c0 < K, live1 = c1 < K;
   int rp = 0;
@@ -1961,8 +1959,11 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   }
   __syncthreads();
   // ---- 3. rotations ------------------------------------------------------------
-  // rotation threshold: above the rounding noise of a length-K dot product
-  const T tol = T(8 * max(K, 8)) * Eps<T>::v;
+  // rotation threshold: above the rounding noise of a length-K dot product.  Half of it in
+  // VG, whose u_i = M v_i / sigma_i take sigma_j (v_j^T v_i) / sigma_i of the larger ones
+  // (K = 128, sigma_r = 1e-8 ||M||: U^T U off by 7.5e-6, 1.7e-5 with the whole; 0.3 ms of
+  // the 147 of a tiled QR of 6 x 6 tiles of 256).
+  const T tol = T((VG ? 4 : 8) * max(K, 8)) * Eps<T>::v;
   const T itol = T(1) / tol;
   // The rounds run the round-robin schedule cyclically and stop once n2 - 1
   // consecutive rounds (every pair once, from any starting round) rotated

@@ -86,8 +86,9 @@ def test_parts_of_a_truncated_sum(torch_gpu, fa, k, eps, decay):
 
 
 def test_left_vectors_of_large_cores(torch_gpu, fa):
-    """Above 64 columns, sigma_r = 1e-8 of the norm: orthogonal to 9.0e-6 in the mean of 48 additions with
-    the core's QR run to its end, to 1.7e-5 when it stops at u ||M||_F and 2.8e-5 at 1e-11 ||M||_F."""
+    """Above 64 columns, sigma_r = 1e-8 of the norm: orthogonal to 7.5e-6 in the mean of 48 additions with
+    the core's QR stopped at u ||M||_F and its rotations at 4 K u, to 1.7e-5 with 8 K u, and to 2.8e-5
+    with the QR stopped at 1e-11 ||M||_F."""
     rng = np.random.default_rng(7)
     out, _ = _add(torch_gpu, fa, [_operands(rng, 200, 150, 64, 64, 0.5) for _ in range(48)], "float64", 1e-8,
                   "rounded_addition")
