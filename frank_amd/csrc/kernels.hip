@@ -92,9 +92,28 @@ __device__ __forceinline__ T wave_sum(T v) {
   v += xor16(v);
   return half_sum(v);
 }
-// e with |v| = f 2^e, f in [1/2, 1); 0 for zero, infinity and NaN.  x 2^e.
-__device__ __forceinline__ int exponent_of(double v) { return __builtin_amdgcn_frexp_exp(v); }
-__device__ __forceinline__ int exponent_of(float v) { return __builtin_amdgcn_frexp_expf(v); }
+__device__ __forceinline__ unsigned umax32(unsigned a, unsigned b) { return a > b ? a : b; }
+// largest of the 64 lanes' values, in every lane
+__device__ __forceinline__ unsigned wave_umax(unsigned v) {
+  v = umax32(v, (unsigned)dpp_i<0xB1>((int)v));
+  v = umax32(v, (unsigned)dpp_i<0x4E>((int)v));
+  v = umax32(v, (unsigned)dpp_i<0x141>((int)v));
+  v = umax32(v, (unsigned)dpp_i<0x140>((int)v));
+  v = umax32(v, (unsigned)swz16_i((int)v));
+  const auto r = __builtin_amdgcn_permlane32_swap((int)v, (int)v, false, false);
+  return umax32((unsigned)r[0], (unsigned)r[1]);
+}
+// The word of |v| that orders by magnitude, and e with |v| in [2^(e-1), 2^e) from it (the
+// least exponent for a denormal number, 0 for zero, infinity and NaN)
+__device__ __forceinline__ unsigned magnitude(double v) { return (unsigned)__double2hiint(v) & 0x7fffffffu; }
+__device__ __forceinline__ unsigned magnitude(float v) { return __float_as_uint(v) & 0x7fffffffu; }
+template <typename T>
+__device__ __forceinline__ int exponent_of(unsigned w) {
+  constexpr int F = sizeof(T) == 8 ? 20 : 23, B = sizeof(T) == 8 ? 1022 : 126;
+  const int e = (int)(w >> F);
+  return (w == 0 || e == 2 * B + 3) ? 0 : e - B;
+}
+// x 2^e
 __device__ __forceinline__ double scaled(double x, int e) { return __builtin_ldexp(x, e); }
 __device__ __forceinline__ float scaled(float x, int e) { return __builtin_ldexpf(x, e); }
 // largest of the 64 lanes' values (not NaN), in every lane
@@ -1083,10 +1102,10 @@ __global__ __launch_bounds__(W * 64) void qr_kernel(Src items) {
   constexpr int kSafeExp = sizeof(T) == 8 ? 400 : 39;
 #pragma unroll
   for (int q = 0; q < CPW; ++q) {
-    T mx = T(0);
+    unsigned mx = 0;
 #pragma unroll
-    for (int t = 0; t < MR; ++t) mx = fmax(mx, fabs(a[q][t]));
-    ex[q] = __builtin_amdgcn_readfirstlane(exponent_of(wave_max(mx)));
+    for (int t = 0; t < MR; ++t) mx = umax32(mx, magnitude(a[q][t]));
+    ex[q] = exponent_of<T>(__builtin_amdgcn_readfirstlane(wave_umax(mx)));
     if (ex[q] > -kSafeExp && ex[q] < kSafeExp) ex[q] = 0;
     if (ex[q] != 0) {
 #pragma unroll
@@ -1161,16 +1180,20 @@ __global__ __launch_bounds__(W * 64) void qr_kernel(Src items) {
 #pragma unroll
   for (int q = 0; q < CPW; ++q) {
     const int c = q * W + w;
+    if (ex[q] != 0) {
+#pragma unroll
+      for (int t = 0; t < MR; ++t)
+        if (lane + 64 * t <= c) a[q][t] = scaled(a[q][t], ex[q]);  // R's rows
+    }
     if (c < K) {
 #pragma unroll
       for (int t = 0; t < MR; ++t) {
         const int row = lane + 64 * t;
         if (row < m && row > c && c < nref) Y[row * it.y_rs + c * it.y_cs] = a[q][t];
-        const T rv = (ex[q] != 0) ? scaled(a[q][t], ex[q]) : a[q][t];
         if (it.r_upper_only) {
-          if (row <= c && row < nref) Rb[(int64_t)(kp + row) * ldr + c] = rv;
+          if (row <= c && row < nref) Rb[(int64_t)(kp + row) * ldr + c] = a[q][t];
         } else if (row < nref) {
-          Rb[(int64_t)(kp + row) * ldr + c] = (row <= c) ? rv : T(0);
+          Rb[(int64_t)(kp + row) * ldr + c] = (row <= c) ? a[q][t] : T(0);
         } else if (row < K) {
           Rb[(int64_t)(kp + row) * ldr + c] = T(0);
         }
@@ -1628,7 +1651,6 @@ __device__ __forceinline__ void jacobi_rotation(float al, float be, float ga, fl
   c = __builtin_amdgcn_rsqf(1.0f + t * t);
   s = c * t;
 }
-__device__ __forceinline__ unsigned umax32(unsigned a, unsigned b) { return a > b ? a : b; }
 // max over the 64 / GL groups of a wave of a value uniform over each group
 template <int GL>
 __device__ __forceinline__ unsigned groups_umax(unsigned k) {
