@@ -1594,9 +1594,11 @@ void launch_tri_extract(const T* src, int64_t rs, int64_t cs, T* dst, int64_t ld
 //      its best remaining column through LDS, so a step costs one barrier.  It
 //      stops at the numerical rank rp, once the trailing block E is below the floor
 //      at which the rotations take a column for zero (u ||M||_F, u the unit
-//      roundoff, or less for a smaller eps).  Stopping earlier, at a share of the
-//      truncation accuracy, would leave the sum U S V alone but move the kept
-//      singular values, by ||E||^2 / 2 sigma.
+//      roundoff, or less for a smaller eps) or, for a truncation at eps, once
+//      ||E||^2 <= u (eps / sqrt(K)) ||M||_F^2: the truncation drops E whole, and a
+//      kept singular value, above eps ||M||_F / sqrt(K), moves by ||E||^2 / 2 sigma,
+//      at most u / 2 ||M||_F.  (1e-3 eps ||M||_F is the upper limit: in FP32 the floor
+//      decides.)
 //   3. One-sided Jacobi on R^T (K x rp), whose graded rows converge in few sweeps
 //      (Drmac-Veselic), a round-robin schedule, one barrier a round.  The
 //      rotations also turn Q into the left vectors.  VG (FP64, K > 64: the second
@@ -1883,7 +1885,10 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   if (it.fixed_rank < 0 && it.eps > 0.0) fl = fmin(fl, static_cast<T>(it.eps / (16.0 * sqrt((double)K))));
   // (an infinity in M makes fro2 one: nothing is small against it, and what it meets
   // becomes NaN)
-  const T tiny = fl * fl * fro2, delta2 = !isfinite(fro2) ? T(0) : tiny;
+  T fd2 = fl * fl;
+  if (it.fixed_rank < 0 && it.eps > 0.0)
+    fd2 = fmax(fd2, static_cast<T>(fmin(1e-6 * it.eps * it.eps, (double)Eps<T>::v * it.eps / sqrt((double)K))));
+  const T tiny = fl * fl * fro2, delta2 = !isfinite(fro2) ? T(0) : fd2 * fro2;
   // ---- 2. pivoted QR, columns in registers -----------------------------------
   bool live0 = c0 < K, live1 = c1 < K;
   int rp = 0;
@@ -1981,11 +1986,11 @@ __global__ __launch_bounds__(KMAX / 2 * GL) void svd_kernel(Src items) {
   }
   __syncthreads();
   // ---- 3. rotations ------------------------------------------------------------
-  // rotation threshold: above the rounding noise of a length-K dot product.  Half of it in
-  // VG, whose u_i = M v_i / sigma_i take sigma_j (v_j^T v_i) / sigma_i of the larger ones
-  // (K = 128, sigma_r = 1e-8 ||M||: U^T U off by 7.5e-6, 1.7e-5 with the whole; 0.3 ms of
-  // the 147 of a tiled QR of 6 x 6 tiles of 256).
-  const T tol = T((VG ? 4 : 8) * max(K, 8)) * Eps<T>::v;
+  // rotation threshold: above the rounding noise of a length-K dot product.  A quarter of
+  // it in VG, whose u_i = M v_i / sigma_i take sigma_j (v_j^T v_i) / sigma_i of the larger
+  // ones (K = 128, sigma_r = 1e-8 ||M||: U^T U off by 3e-6, 1.7e-5 with the whole; 0.5 ms
+  // of the 145 of a tiled QR of 6 x 6 tiles of 256).
+  const T tol = T((VG ? 2 : 8) * max(K, 8)) * Eps<T>::v;
   const T itol = T(1) / tol;
   // The rounds run the round-robin schedule cyclically and stop once n2 - 1
   // consecutive rounds (every pair once, from any starting round) rotated

@@ -86,15 +86,15 @@ def test_parts_of_a_truncated_sum(torch_gpu, fa, k, eps, decay):
 
 
 def test_left_vectors_of_large_cores(torch_gpu, fa):
-    """Above 64 columns, sigma_r = 1e-8 of the norm: orthogonal to 7.5e-6 in the mean of 48 additions with
-    the core's QR stopped at u ||M||_F and its rotations at 4 K u, to 1.7e-5 with 8 K u, and to 2.8e-5
-    with the QR stopped at 1e-11 ||M||_F."""
+    """Above 64 columns, sigma_r = 1e-8 of the norm: u_i = M v_i / sigma_i are as orthogonal as the v_i leave
+    them.  Mean of 48 additions: 9.0e-6 with every column of the core rotated to 8 K u; 1.7e-5 with the
+    columns below u ||M||_F left out, 2.8e-5 below 1e-11 ||M||_F; a few 1e-6 with the rotations to 2 K u."""
     rng = np.random.default_rng(7)
     out, _ = _add(torch_gpu, fa, [_operands(rng, 200, 150, 64, 64, 0.5) for _ in range(48)], "float64", 1e-8,
                   "rounded_addition")
     err = [np.abs((U.T @ U).astype(np.float64) - np.eye(U.shape[1])).max() for U, _, _ in out]
     print(f"left vectors: {np.mean(err):.3e}", flush=True)
-    assert np.mean(err) <= 1.3e-5
+    assert np.mean(err) <= 9e-6
 
 
 @pytest.mark.parametrize("m,n,k1,k2", [(64, 60, 5, 3), (64, 64, 16, 9), (128, 100, 17, 16), (256, 200, 16, 16),
