@@ -1609,10 +1609,10 @@ void launch_tri_extract(const T* src, int64_t rs, int64_t cs, T* dst, int64_t ld
 // traffic of the rotations.  Launch averages, before (one array read with scalar
 // strided columns, norms recomputed per QR step, a serial pivot search, K full
 // columns; a register kernel for K <= 16 and FP64 K <= 32) -> now: FP64 K <= 16,
-// 778 cores 69 -> 35 us; FP64 K <= 32, 590 cores 214 -> 52 us; FP64 K <= 64, 165
-// cores 1.78 -> 0.69 ms; FP64 K <= 128, 5 cores 2.84 -> 0.95 ms; FP32 K <= 16, 672
-// cores 22.6 -> 18.5 us; FP32 K <= 64, 1231 cores 1.29 -> 0.51 ms; FP32 K <= 128,
-// 817 cores 5.66 -> 1.45 ms.
+// 778 cores 69 -> 36 us; FP64 K <= 32, 590 cores 214 -> 52 us; FP64 K <= 64, 165
+// cores 1.78 -> 0.68 ms; FP64 K <= 128, 5 cores 2.84 -> 1.08 ms; FP32 K <= 16, 672
+// cores 22.6 -> 19.1 us; FP32 K <= 64, 1231 cores 1.29 -> 0.53 ms; FP32 K <= 128,
+// 817 cores 5.66 -> 1.61 ms.
 // ---------------------------------------------------------------------------
 template <typename T, int N>
 struct LdsVec {

@@ -25,16 +25,16 @@
 // FP64 only: in FP32 the compact WY form (T, and one more rounding of T^T W) left an
 // error of the sum of 2.2e-7 at m = 256, K = 32, singular values 10^(-i/2), against
 // 1.8e-7 with a reflector at a time, which the additions in FP32 keep.
-// Measured, FP64, QR of both panels and basis update, us, these kernels / the
-// unblocked ones (a reflector at a time over the whole panel, two barriers each):
+// Measured, QR of both panels and basis update with every column kept, us, these
+// kernels / the unblocked ones (a reflector at a time over the whole panel, two barriers
+// each):
 //   m    K    additions   QR             update
-//   64   16   40          13.0 / 19.8    7.0 / 9.0
-//   64   128  165         78.9 / 323     25.4 / 121
-//   128  32   300         54.8 / 73.2    20.4 / 40.6
-//   256  16   40          19.6 / 24.8    10.0 / 11.4
-//   256  64   165         132  / 184     27 / 101
-//   256  128  4           190  / 254     60 / 32  (the one update that is slower: few
-//                                        waves, and a panel's loads in a chain)
+//   64   16   40          12.5 / 18.6    5.8 / 14.2
+//   64   128  165         95.0 / 325     23.1 / 123
+//   128  32   300         56.7 / 71.8    22.9 / 77.4
+//   256  16   40          18.9 / 23.6    9.0 / 18.6
+//   256  64   165         146 / 191      78.1 / 182
+//   256  128  4           202 / 264      105 / 289
 #include <hip/hip_runtime.h>
 
 #include <stdexcept>
@@ -155,8 +155,8 @@ __device__ __forceinline__ double rsqrt_of(double x) {
 }
 __device__ __forceinline__ double inv_of(double x) { return d64::rcp2(x); }
 
-// Squared norm at and below which a pivot column counts as zero, of a column scaled to
-// a largest entry in [1/2, 1).
+// Squared norm at and below which a pivot column counts as zero: of a column whose
+// largest entry was 2^-400 or more, so 1e-30 of its norm.
 constexpr double kZeroNorm2 = 1e-300;
 
 // A wave's share of a panel: tiles x (tile t is tile t RW + rw of the column), the
@@ -333,6 +333,7 @@ __global__ __launch_bounds__(64 * NP * RW, (NT == 4 && NP == 8) ? 4 : 1) void lr
   __shared__ T Ts[NP > 1 ? 2 : 1][NP > 1 ? 256 : 1];
   __shared__ T Wp[RW > 1 ? 256 * NP * RW : 1];  // partial products of the row shares
   __shared__ T ex[RW > 1 ? 64 * RW : 1];
+  __shared__ int ses[16 * NP * RW];  // exponents of the columns' scales
   // the sum of the RW shares of a 16 x 16 product
   auto rw_sum = [&](v4 z) {
     if constexpr (RW > 1) {
@@ -443,10 +444,9 @@ __global__ __launch_bounds__(64 * NP * RW, (NT == 4 && NP == 8) ? 4 : 1) void lr
       if constexpr (RW > 1) __syncthreads();  // Wp free
     }
   }
-  // ---- every column to a largest entry in [1/2, 1), by a power of two ----------------
+  // ---- columns of extreme norm to a largest entry in [1/2, 1), by a power of two ------
   // Reflectors and T do not depend on the columns' scales, R takes them back: norms of
-  // any size neither overflow nor fall under `tiny`, which is then relative to the column.
-  int se = 0;
+  // any size neither overflow nor fall under kZeroNorm2.
   {
     T mx = T(0);
 #pragma unroll
@@ -460,11 +460,17 @@ __global__ __launch_bounds__(64 * NP * RW, (NT == 4 && NP == 8) ? 4 : 1) void lr
 #pragma unroll
       for (int r = 0; r < RW; ++r) mx = fmax(mx, Wp[256 * (w * RW + r) + li]);
     }
-    se = exponent_of(mx);
+    int se = exponent_of(mx);
+    se = (se > -400 && se < 400) ? 0 : se;
+    if (lr == 0) ses[16 * wid + li] = se;  // (a register held through the panels would spill)
+    // (scaling every panel spills at NT = 8: 199 us instead of 144 at 256 rows, 64 columns,
+    // 165 additions; at the others it costs nothing)
+    if (NT != 8 || __any(se != 0)) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[t][e] = scaled(x[t][e], -se);
+        for (int e = 0; e < 4; ++e) x[t][e] = scaled(x[t][e], -se);
+    }
   }
   // ---- factorization, panel by panel ------------------------------------------------
   const Buf<T> Y(it.Y), Tg(it.tau);
@@ -511,7 +517,7 @@ __global__ __launch_bounds__(64 * NP * RW, (NT == 4 && NP == 8) ? 4 : 1) void lr
       for (int e = 0; e < 4; ++e) {
         const int row = 4 * lr + e;
         const T rv = (row < li) ? p.top[e] : (row == li ? p.rd : T(0));
-        Rb.store(at<T>(owner && own && j0 + row < K, kp + j0 + row, ldr, c, 1), (row < lim) ? scaled(rv, se) : T(0));
+        Rb.store(at<T>(owner && own && j0 + row < K, kp + j0 + row, ldr, c, 1), (row < lim) ? scaled(rv, ses[16 * wid + li]) : T(0));
         p.top[e] = (li >= lim || row < li) ? T(0) : (row == li ? T(1) : p.top[e] * p.inv);
       }
 #pragma unroll
@@ -572,7 +578,7 @@ __global__ __launch_bounds__(64 * NP * RW, (NT == 4 && NP == 8) ? 4 : 1) void lr
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int row = j0 + 4 * lr + e;
-          Rb.store(at<T>(own && row < K, kp + row, ldr, c, 1), (row < nref) ? scaled(top[e], se) : T(0));
+          Rb.store(at<T>(own && row < K, kp + row, ldr, c, 1), (row < nref) ? scaled(top[e], ses[16 * wid + li]) : T(0));
         }
       }
     }
