@@ -135,3 +135,42 @@ def test_right_vectors_of_small_cores(torch_gpu, fa, k, lra, eps):
         assert np.abs((U.T @ U).astype(np.float64) - np.eye(r)).max() <= 16 * max(K, 8) * u
         tail = np.linalg.norm(np.linalg.svd(D.astype(np.float64), compute_uv=False)[r:])
         assert _norm(D - U @ (S @ V)) <= tail * (1 + 1e-6) + 8 * K * u * _norm(D)
+
+
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("m,k", [(64, 12), (128, 8), (256, 16), (256, 24), (256, 40), (400, 16)])
+def test_chain_of_fast_additions(torch_gpu, fa, dtype, m, k):
+    """Twelve additions from the space that C spans, as a fixed-rank block LU makes them: each sum has the rank
+    that is kept, so what is left is the rounding of twelve additions.  It does not grow with the loss of
+    orthogonality that each passes on to the next (one projection in blocks of 16 left errors of 1e-3 in FP32
+    and bases 1e-7 from orthonormal in FP64)."""
+    torch = torch_gpu
+    rng = np.random.default_rng(5)
+    u, dt, cap, steps = np.finfo(dtype).eps, getattr(torch, dtype), 128, 12
+    up = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to("cuda", dt)
+    wide = lambda x: x.double().cpu().numpy().astype(np.longdouble)
+    q = lambda r, c: np.linalg.qr(rng.standard_normal((r, c)))[0]
+    s = np.diag(10.0 ** (-0.2 * np.arange(k)))
+    spaces = [(q(m, k), q(m, k)) for _ in range(4)]
+    As, Ds, size = [], [], []
+    for a, b in spaces:
+        U, S, V = (torch.zeros(x, dtype=dt, device="cuda") for x in ((m, cap), (cap, cap), (cap, m)))
+        U[:, :k], S[:k, :k], V[:k] = up(a), up(s), up(b.T)
+        As.append((U, S, V, k))
+        Ds.append(wide(U[:, :k]) @ (wide(S[:k, :k]) @ wide(V[:k])))
+    for _ in range(steps):
+        Bs = [(up(a @ q(k, k)), up(s), up((b @ q(k, k)).T)) for a, b in spaces]
+        Ds = [D + wide(U) @ (wide(S) @ wide(V)) for D, (U, S, V) in zip(Ds, Bs)]
+        assert list(fa.lr_add_batched(As, Bs, eps=0.0, lra="fast_rounded_addition", cap=cap)) == [k] * len(As)
+    # rounding of each addition (some sqrt(K) u of the norms of its operands, K = 2 k), and the operands' own,
+    # which lie in C's space to u only; above 64 columns FP64 forms u_i = M v_i / sigma_i, and U S V is off by
+    # what the v_i are from orthogonal, the rotation threshold 2 K u
+    lim = 4 * np.sqrt(2 * k) * u + (2 * 2 * k * u if dtype == "float64" and 2 * k > 64 else 0.0)
+    for (U, S, V, _), D in zip(As, Ds):
+        err = _norm(D - wide(U[:, :k]) @ (wide(S[:k, :k]) @ wide(V[:k]))) / _norm(D)
+        print(f"chain {dtype} m={m} k={k}: {err:.2e}", flush=True)
+        assert err <= steps * lim
+        # FP64 up to 256 rows projects twice: the bases stay at the rotation threshold 8 max(K, 8) u, left and right
+        if dtype == "float64" and m <= 256 and 2 * k <= 64:
+            for W in (wide(U[:, :k]), wide(V[:k]).T):
+                assert np.abs((W.T @ W).astype(np.float64) - np.eye(k)).max() <= 4 * 8 * max(2 * k, 8) * u
