@@ -1,7 +1,7 @@
-"""Blocked QR and basis update of the batched low-rank addition at the edges of their
-tiles (16 rows, 16 columns), of their variants (64, 128, 256 rows; 16, 32, 64, 128
-columns; past them the unblocked kernels), for tiles smaller than the columns added,
-both layouts of the bases, and both additions (rounded; fast, which projects first)."""
+"""QR and basis update of the batched low-rank addition at the edges of the blocked FP64
+kernels' tiles (16 rows, 16 columns), of their variants (64, 128, 256 rows; 16, 32, 64, 128
+columns; past them, and in FP32, the unblocked kernels), for tiles smaller than the columns
+added, both layouts of the bases, and both additions (rounded; fast, which projects first)."""
 import numpy as np
 import pytest
 
@@ -76,8 +76,8 @@ def test_tile_edges(torch_gpu, fa, dtype, lra, case):
 
 @pytest.mark.parametrize("dtype", ["float64", "float32"])
 def test_both_routes_of_a_tall_narrow_batch(torch_gpu, fa, dtype):
-    """129 to 256 rows and at most 32 columns: up to 128 additions take the blocked kernels, more
-    the unblocked ones; the same additions give the same sums either way."""
+    """129 to 256 rows and at most 32 columns: up to 128 additions in FP64 take the blocked kernels, more
+    (and FP32 always) the unblocked ones; the same additions give the same sums either way."""
     torch = torch_gpu
     rng = np.random.default_rng(3)
     u, dt, k, cap = np.finfo(dtype).eps, getattr(torch, dtype), 9, 32
